@@ -1,0 +1,71 @@
+"""Decode attention over ragged batches with automatic splits: the splits
+follow the sequences' lengths (one chunk for the whole call, as many splits as
+a sequence needs), in every mode, against the fp64 oracle within
+zs_testutil.attention_tolerance, and compressed against dense bit for bit where
+both cut the same pieces."""
+import numpy as np
+import pytest
+
+from test_gpu_attention import _check, _run
+
+pytestmark = pytest.mark.gpu
+
+
+def _lens(B, T, seed):
+    rng = np.random.default_rng(seed)
+    lens = rng.integers(0, T + 1, B)
+    lens[0], lens[-1] = T, 0
+    return [int(v) for v in lens]
+
+
+CASES = [
+    (2, 500, [500, 1]),                      # one long, one token
+    (3, 1100, [0, 1100, 0]),                 # all pieces in one sequence
+    (4, 2000, [2000] * 4),                   # equal lengths: the even split
+    (4, 2000, [0, 0, 0, 0]),                 # no tokens at all
+    (5, 640, [640, 16, 17, 15, 9999]),       # band edges, a length past the cache
+    (64, 260, _lens(64, 260, 1)),            # one wave's lanes of lengths
+    (65, 260, _lens(65, 260, 2)),            # one more than a wave holds
+    (130, 150, _lens(130, 150, 3)),          # three chunks of lengths
+]
+
+
+@pytest.mark.parametrize("B,T,lens", CASES)
+@pytest.mark.parametrize("retiled", [False, True])
+def test_ragged_head_major(torch_cuda, B, T, lens, retiled):
+    used = [min(v, T) for v in lens]
+    res = _run(torch_cuda, B, T, 2, 8, seqlens=used, splits=0, seed=B, retiled=retiled)
+    # the dense kernel cuts the same pieces where its split count is the same
+    # (short sequences: the minimum split length decides in both)
+    _check(res, used, exact=B <= 5 and T < 1000)
+
+
+@pytest.mark.parametrize("B,T,lens", CASES)
+def test_ragged_token_major(torch_cuda, B, T, lens):
+    used = [min(v, T) for v in lens]
+    _check(_run(torch_cuda, B, T, 8, 16, seqlens=used, splits=0, seed=B + 1, retiled=True,
+                layout="token_major"), used, exact=False)
+
+
+def test_ragged_large_grid(torch_cuda):
+    # one wave per item in the head-major kernel (>= 2048 items), the last
+    # workgroups past the last piece
+    lens = [4096, 100, 2048, 3000, 1, 0, 4000, 511] * 2
+    _check(_run(torch_cuda, 16, 4096, 8, 32, seqlens=lens, splits=0, seed=9, retiled=True), lens,
+           exact=False)
+
+
+def test_ragged_lengths_past_the_cache_are_clamped(torch_cuda):
+    import zipserv_asplos26_amd.attention as za
+    torch = torch_cuda
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    x = [torch.randn(3, 600, 8, 128, device="cuda", generator=g).to(torch.bfloat16) for _ in "kv"]
+    q = torch.randn(3, 1, 64, 128, device="cuda", generator=g).to(torch.bfloat16)
+    for layout in ("by_kv_head", "token_major"):
+        k, v = (za.compress_kv(t, layout=layout, retiled=True) for t in x)
+        outs = [za.flash_attn_with_kvcache_zipserv(
+            q, k, v, 8, 600, torch.tensor(s, dtype=torch.int32, device="cuda"))
+            for s in ([600, 0, 77], [1 << 30, -5, 77])]
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
