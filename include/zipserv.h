@@ -246,6 +246,23 @@ int zs_compress_retiled_guess_gpu(void* stream, const uint16_t* d_input, int M, 
 int zs_compress_retiled_exps_gpu(void* stream, const uint16_t* d_input, int M, int K,
                                  const int32_t* d_top_exponents, const int32_t* d_eoff,
                                  const uint8_t* d_tmp, uint8_t* d_exps);
+/* zs_compress_retiled_auto_gpu / _exps_gpu over a dense cache
+ * [batch][tokens][heads][head_dim] (16-byte aligned, head_dim % 64 == 0)
+ * instead of the padded matrix of its layout
+ * (bench_zipserv_decode_attention.py:337-364): group_rows rows per (batch,
+ * head) (ZS_LAYOUT_HEAD_MAJOR, >= tokens) or per batch entry
+ * (ZS_LAYOUT_TOKEN_MAJOR, >= tokens * heads), a multiple of 16, the rows past
+ * the cache's own zero.  The bytes are those of the padded matrix; no copy of
+ * the cache is made. */
+int zs_compress_retiled_kv_gpu(void* stream, const uint16_t* d_cache, int layout, int batch,
+                               int tokens, int heads, int head_dim, int group_rows, int rule,
+                               uint64_t* d_hist, int32_t* d_top, uint8_t* d_work,
+                               uint8_t* d_fixed, int32_t* d_counts, int32_t* d_eoff,
+                               int64_t* d_total, uint8_t* d_tmp);
+int zs_compress_retiled_kv_exps_gpu(void* stream, const uint16_t* d_cache, int layout, int batch,
+                                    int tokens, int heads, int head_dim, int group_rows,
+                                    const int32_t* d_top_exponents, const int32_t* d_eoff,
+                                    const uint8_t* d_tmp, uint8_t* d_exps);
 /* Canonical TCA-TBE streams -> re-tiled, same two phases (window start_exp). */
 int zs_retile_triple_bitmap_count_gpu(void* stream, const uint8_t* SignMantissa,
                                       const uint16_t* CompressedFull, const uint64_t* Bitmap1,

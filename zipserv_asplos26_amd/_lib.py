@@ -70,6 +70,8 @@ SIGNATURES = {
     "zs_compress_retiled_guess_gpu": (C.c_int, [_p, _p, C.c_int, C.c_int, C.c_int, _p, _p, _p, _p,
                                                 _p, _p, _p, _p, _p]),
     "zs_compress_retiled_exps_gpu": (C.c_int, [_p, _p, C.c_int, C.c_int, _p, _p, _p, _p]),
+    "zs_compress_retiled_kv_gpu": (C.c_int, [_p, _p] + [C.c_int] * 7 + [_p] * 8),
+    "zs_compress_retiled_kv_exps_gpu": (C.c_int, [_p, _p] + [C.c_int] * 6 + [_p] * 4),
     "zs_retile_triple_bitmap_count_gpu": (
         C.c_int, [_p, _p, _p, _p, _p, _p, _p, _p, C.c_int, C.c_int, _p, _p, _p]),
     "zs_retile_triple_bitmap_emit_gpu": (

@@ -15,7 +15,8 @@ from typing import Optional
 
 from . import _lib
 from ._lib import check, lib
-from .codec import ZipservRetiled, _check_cuda, _dptr, _stream, _torch, compress, compress_retiled
+from .codec import (ZipservRetiled, _check_cuda, _dptr, _stream, _torch, compress, compress_retiled,
+                    compress_retiled_kv)
 
 # flash_attn_interface.py:38-43 (_ZIPSERV_LAYOUT_IDS)
 LAYOUT_IDS = {"by_kv_head": _lib.ZS_LAYOUT_HEAD_MAJOR, "dense": _lib.ZS_LAYOUT_TOKEN_MAJOR,
@@ -105,12 +106,44 @@ def decompress_to_batched_paged_kv(comp, batch_size_cache: int, kv_heads: int, h
         batch_size_cache * (padded // page_block_size), page_block_size, kv_heads, head_dim)
 
 
+def _kv_group(x, layout, page_block_size):
+    """(rows per group, logical rows) of the padded matrix that the pad_*
+    helpers build of a (B, T, Hkv, D) cache."""
+    B, T, H, _ = x.shape
+    if layout == "by_kv_head":
+        rph = (T + 63) // 64 * 64
+        return rph, B * H * rph
+    if layout == "paged":
+        return (T + page_block_size - 1) // page_block_size * page_block_size * H, B * T * H
+    return (T * H + 63) // 64 * 64, B * T * H
+
+
+def _reads_in_place(x, layout, page_block_size):
+    """Whether the re-tiled encoder can read the cache itself: contiguous and
+    16-byte aligned bf16 on the GPU, whole 64-dim column tiles, and 16-row
+    bands and 64-row tiles that do not cross the padded matrix's groups.
+    Everything else goes through the padded copy."""
+    torch = _torch()
+    if not (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == torch.bfloat16
+            and x.dim() == 4 and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and x.numel() > 0 and x.shape[3] % 64 == 0
+            and layout in ("by_kv_head", "token_major", "dense", "paged")):
+        return False
+    if layout == "paged" and page_block_size <= 0:
+        return False
+    return _kv_group(x, layout, page_block_size)[0] % 64 == 0
+
+
 def compress_kv(x, layout: str = "by_kv_head", retiled: bool = False,
                 page_block_size: int = 16):
     """Pack a (B, T, Hkv, D) bf16 cache and compress it on the GPU into the
     canonical streams (ZipservCompressed) or the re-tiled layout
     (ZipservRetiled).  layout "paged" pads each sequence to whole pages of
-    page_block_size tokens (token-major rows)."""
+    page_block_size tokens (token-major rows).  The re-tiled encoder reads a
+    contiguous cache in place (compress_retiled_kv): the padded, transposed
+    copy took 53 of 130 us of the GPU's time per 67 MB cache."""
+    if retiled and _reads_in_place(x, layout, page_block_size):
+        return compress_retiled_kv(x, layout, *_kv_group(x, layout, page_block_size))
     if layout == "by_kv_head":
         mat, logical_rows, _ = pad_batched_kv_prefix_by_kv_head(x)
     elif layout in ("token_major", "dense"):

@@ -490,19 +490,25 @@ def _retiled_alloc(rows, cols, total, dev):
     return fixed, exps, nrec
 
 
-def _retiled_encode(input, window, guess=None):
+def _retiled_encode(input, window, guess=None, kv=None):
     """First phase of the re-tiled GPU encoder on the current stream: the
     window, the fixed parts, the per-record outlier counts and offsets, and
     the outlier bytes in per-record slots; the outlier total and the window
     land in one int64 [5] tensor (`meta`) that the host reads to size the
     exponent stream.  Under a window rule, `guess` (int32 [7] on the device,
     e.g. the previous matrix's window) replaces the sampled guess; the bytes
-    are the same either way.  Returns the state _retiled_finish takes."""
+    are the same either way.  `kv` (layout id, batch, tokens, heads, head_dim,
+    group_rows; zs_compress_retiled_kv_gpu): `input` is a dense cache, encoded
+    as the padded matrix of that layout.  Returns the state _retiled_finish
+    takes."""
     torch = _torch()
     _check_cuda(input, "input", torch.bfloat16)
-    if input.dim() != 2:
+    if kv is not None:
+        rows, cols = kv[1] * (kv[3] if kv[0] == _lib.ZS_LAYOUT_HEAD_MAJOR else 1) * kv[5], kv[4]
+    elif input.dim() != 2:
         raise ValueError("input must be 2D")
-    rows, cols = input.shape
+    else:
+        rows, cols = input.shape
     if rows % 64 or cols % 64:
         raise ValueError("rows and cols must be padded to multiples of 64")
     L = lib()
@@ -524,7 +530,12 @@ def _retiled_encode(input, window, guess=None):
         rule = _lib.ZS_WINDOW_KV if window == "kv" else _lib.ZS_WINDOW_WEIGHTS
         work = torch.empty(_lib.ZS_RETILED_AUTO_WORK_BYTES, dtype=torch.uint8, device=dev)
         # 64-bit bins: the re-tiled layout takes matrices past 2^31 elements.
-        if guess is not None:
+        if kv is not None:
+            check("zs_compress_retiled_kv_gpu",
+                  L.zs_compress_retiled_kv_gpu(st, _dptr(input), *kv, rule, _dptr(counts),
+                                               _dptr(top), _dptr(work), _dptr(fixed), _dptr(cnt),
+                                               _dptr(eoff), _dptr(total), _dptr(tmp)))
+        elif guess is not None:
             _check_cuda(guess, "guess", torch.int32)
             check("zs_compress_retiled_guess_gpu",
                   L.zs_compress_retiled_guess_gpu(st, _dptr(input), rows, cols, rule, _dptr(guess),
@@ -543,7 +554,7 @@ def _retiled_encode(input, window, guess=None):
                                               _dptr(fixed), _dptr(cnt), _dptr(eoff),
                                               _dptr(total), _dptr(tmp)))
     return dict(input=input, rows=rows, cols=cols, nrec=nrec, meta=meta, top=top, eoff=eoff,
-                fixed=fixed, tmp=tmp)
+                fixed=fixed, tmp=tmp, kv=kv)
 
 
 def _retiled_finish(s, host_meta, logical_rows, logical_cols, layout) -> ZipservRetiled:
@@ -557,10 +568,13 @@ def _retiled_finish(s, host_meta, logical_rows, logical_cols, layout) -> Zipserv
     # every byte is written by the compaction, the slack bytes as zeros
     exps = torch.empty(tot + _lib.ZS_STREAM_SLACK_BYTES, dtype=torch.uint8,
                        device=s["input"].device)
-    check("zs_compress_retiled_exps_gpu",
-          lib().zs_compress_retiled_exps_gpu(_stream(), _dptr(s["input"]), rows, cols,
-                                             _dptr(s["top"]), _dptr(s["eoff"]), _dptr(s["tmp"]),
-                                             _dptr(exps)))
+    args = [_dptr(s["top"]), _dptr(s["eoff"]), _dptr(s["tmp"]), _dptr(exps)]
+    if s["kv"] is not None:
+        check("zs_compress_retiled_kv_exps_gpu",
+              lib().zs_compress_retiled_kv_exps_gpu(_stream(), _dptr(s["input"]), *s["kv"], *args))
+    else:
+        check("zs_compress_retiled_exps_gpu",
+              lib().zs_compress_retiled_exps_gpu(_stream(), _dptr(s["input"]), rows, cols, *args))
     s.pop("tmp")  # stream-ordered: the allocator reuses it only after the compaction
     return ZipservRetiled(s["fixed"], exps, s["eoff"], rows, cols,
                           rows if logical_rows is None else logical_rows,
@@ -581,6 +595,19 @@ def compress_retiled(input, logical_rows=None, logical_cols=None, layout="by_kv_
     s = _retiled_encode(input, window)
     host = s["meta"].cpu()  # synchronises (sizes the stream)
     return _retiled_finish(s, host, logical_rows, logical_cols, layout)
+
+
+def compress_retiled_kv(cache, layout: str, group_rows: int, logical_rows: int) -> ZipservRetiled:
+    """compress_retiled of a contiguous dense cache (batch, tokens, heads,
+    head_dim) as the padded matrix of `layout` ("by_kv_head", or a token-major
+    one), which is not built: the encoder reads the cache in that order
+    (zs_compress_retiled_kv_gpu).  group_rows: the matrix's rows per (batch,
+    head), or per batch entry."""
+    B, T, H, D = cache.shape
+    lid = _lib.ZS_LAYOUT_HEAD_MAJOR if layout == "by_kv_head" else _lib.ZS_LAYOUT_TOKEN_MAJOR
+    s = _retiled_encode(cache, "kv", kv=(lid, B, T, H, D, group_rows))
+    host = s["meta"].cpu()  # synchronises (sizes the stream)
+    return _retiled_finish(s, host, logical_rows, D, layout)
 
 
 def compress_retiled_many(inputs, window="kv", layout="by_kv_head", lookahead=4) -> list:

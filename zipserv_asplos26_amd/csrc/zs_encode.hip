@@ -97,13 +97,14 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const uint16_t* in, 
 // the arrival counter of the offset scan).
 constexpr int kSampleStrideMin = 32, kSampleChunks = 128, kSampleGroups = 4;
 
-__device__ __forceinline__ int64_t sample_stride(int64_t nchunks) {
+__host__ __device__ __forceinline__ int64_t sample_stride(int64_t nchunks) {
   const int64_t s = (nchunks + kSampleChunks - 1) / kSampleChunks;
   return s > kSampleStrideMin ? s : kSampleStrideMin;
 }
 
 __global__ __launch_bounds__(kHistThreads) void sample_hist_kernel(const uint16_t* in,
                                                                    int64_t nchunks,
+                                                                   uint64_t zeros,
                                                                    uint64_t* slices,
                                                                    uint64_t* zero,
                                                                    int32_t* zero32) {
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(kHistThreads) void sample_hist_kernel(const uint16_
   if (threadIdx.x < 256) {
     uint32_t c = 0;
     for (int k = 0; k < kHistCopies; ++k) c += h[k * kHistPitch + threadIdx.x];
-    slices[256 * blockIdx.x + threadIdx.x] = c;
+    slices[256 * blockIdx.x + threadIdx.x] = c + (blockIdx.x + threadIdx.x == 0 ? zeros : 0);
   }
 }
 
@@ -530,11 +531,15 @@ namespace zs {
 // of 2048, is not sampled; input 16-byte aligned) into `guess`; the per-workgroup
 // sample bins go to `sample` (kSampleGroups x 256), and `zero`
 // (kVerifySlices x 256 entries) and *zero32 (when given) are cleared on the way.
-hipError_t launch_window_sample(hipStream_t st, const uint16_t* in, int64_t numel,
+// `zeros`: elements of the encoded matrix that are not in `in` (zero padding),
+// counted in the sample in proportion.
+hipError_t launch_window_sample(hipStream_t st, const uint16_t* in, int64_t numel, int64_t zeros,
                                 bool weights_rule, uint64_t* sample, uint64_t* zero,
                                 int32_t* guess, int32_t* zero32) {
+  const int64_t nchunks = numel / 2048, stride = sample_stride(nchunks);
+  const int64_t sampled = (nchunks + stride - 1) / stride * 2048;
   hipLaunchKernelGGL(sample_hist_kernel, dim3(kSampleGroups), dim3(kHistThreads), 0, st, in,
-                     numel / 2048, sample, zero, zero32);
+                     nchunks, (uint64_t)((double)zeros * sampled / numel), sample, zero, zero32);
   if (weights_rule)
     hipLaunchKernelGGL((select_weights_kernel<uint64_t, kSampleGroups>), dim3(1), dim3(256), 0, st,
                        sample, nullptr, guess, nullptr, nullptr);

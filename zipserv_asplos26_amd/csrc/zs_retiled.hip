@@ -28,11 +28,48 @@ __device__ __forceinline__ const uint16_t* rec_src_at(const uint16_t* a, int K, 
   const int l = lane_id();
   return a + (band * 16 + (l & 15)) * (int64_t)K + kt * 64 + 32 * h + 8 * (l >> 4);
 }
-__device__ __forceinline__ const uint16_t* rec_src(const uint16_t* a, int K, int64_t rec, int h) {
-  const int KT = K >> 6;
-  const int64_t band = rec / KT;
-  return rec_src_at(a, K, band, (int)(rec - band * KT), h);
-}
+
+// Where the encoders read a record's 16 x 64 elements: lane l's eight of half
+// h of the tile (band, kt).  MatSrc: a row-major matrix.
+struct MatSrc {
+  const uint16_t* a;
+  int K;
+  __device__ __forceinline__ u32x4 load(int64_t band, int kt, int h) const {
+    return *reinterpret_cast<const u32x4*>(rec_src_at(a, K, band, kt, h));
+  }
+};
+
+// n / d for n < 2^31 and d >= 2 by one multiply: m = ceil(2^32 / d) makes
+// mulhi(n, m) the quotient or one more.
+struct FastDiv {
+  uint32_t d, m;  // m == 0: d == 1
+  __device__ __forceinline__ uint32_t div(uint32_t n) const {
+    if (m == 0) return n;
+    const uint32_t q = __umulhi(n, m);
+    return q * d > n ? q - 1 : q;
+  }
+};
+
+// KvSrc: a dense cache [B][T][H][D] read as the matrix that its compressed
+// form stands for -- groups of group_rows rows (head-major: one (b, h) each,
+// token-major: one b), the first `valid` rows of a group from the cache,
+// the rest zeros -- so that no padded, transposed copy is written and read
+// back first.  16-row bands do not cross groups (group_rows % 16 == 0).
+struct KvSrc {
+  const uint16_t* x;
+  FastDiv bands, inner;  // bands per group; groups per batch (head-major: H)
+  int64_t outer_stride, inner_stride, row_stride;  // elements
+  int valid;
+  __device__ __forceinline__ u32x4 load(int64_t band, int kt, int h) const {
+    const uint32_t g = bands.div((uint32_t)band);
+    const int r = (int)((uint32_t)band - g * bands.d) * 16 + (lane_id() & 15);
+    const uint32_t go = inner.div(g);
+    const uint16_t* base = x + go * outer_stride + (g - go * inner.d) * inner_stride + kt * 64 + 32 * h;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(base + min(r, valid - 1) * row_stride +
+                                                    8 * (lane_id() >> 4));
+    return r < valid ? v : u32x4{0, 0, 0, 0};
+  }
+};
 
 // The records a wave of a grid-stride loop visits -- rec = w, w + nw, ...
 // for wave w of nw -- with their (band, K tile) advanced by addition: one
@@ -467,8 +504,8 @@ struct WindowCheck {
   int weights_rule;
 };
 
-template <bool kHist>
-__global__ __launch_bounds__(256) void rfixed_kernel(const uint16_t* a, int M, int K,
+template <bool kHist, typename Src>
+__global__ __launch_bounds__(256) void rfixed_kernel(Src src, int M, int K,
                                                      const int32_t* top, uint8_t* fixed,
                                                      int32_t* counts, uint8_t* tmp,
                                                      uint64_t* hist, const int32_t* redo,
@@ -511,8 +548,7 @@ __global__ __launch_bounds__(256) void rfixed_kernel(const uint16_t* a, int M, i
     const int64_t rec = r.rec;
     u32x4 v[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      v[h] = *reinterpret_cast<const u32x4*>(rec_src_at(a, K, r.band, r.kt, h));
+    for (int h = 0; h < 2; ++h) v[h] = src.load(r.band, r.kt, h);
     const RecCodes rc = rec_codes(v, st);
     if constexpr (kHist) {
       // code bit p of element i of half h at bit 3i + h of P[p]; a code's
@@ -577,7 +613,8 @@ constexpr int kCompactRecs = 8;
 // past its slot writes each record straight to global memory as below.
 constexpr int kCompactBuf = kCompactRecs * kExpFast + 16;  // group range + alignment
 
-__global__ __launch_bounds__(256) void rcompact_kernel(const uint16_t* a, int M, int K,
+template <typename Src>
+__global__ __launch_bounds__(256) void rcompact_kernel(Src src, int M, int K,
                                                        const int32_t* top, const int32_t* eoff,
                                                        const uint8_t* __restrict__ tmp,
                                                        uint8_t* __restrict__ exps) {
@@ -663,9 +700,11 @@ __global__ __launch_bounds__(256) void rcompact_kernel(const uint16_t* a, int M,
       slow &= slow - 1;
       u32x4 x[2];
       uint32_t bp[2][3];
+      const int KT = K >> 6;
+      const int64_t band = (r0 + q) / KT;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        x[h] = *reinterpret_cast<const u32x4*>(rec_src(a, K, r0 + q, h));
+        x[h] = src.load(band, (int)(r0 + q - band * KT), h);
         classify8(x[h], st, bp[h][0], bp[h][1], bp[h][2]);
       }
       emit_exps(exps + __builtin_amdgcn_readlane(e0l, q), x, bp);
@@ -720,7 +759,7 @@ int device_cu_count();  // zs_gemm.hip
 // zs_encode.hip: the window guessed from a sample of the input, and the
 // window of a full histogram with a flag saying whether it differs.
 hipError_t launch_window_sample(hipStream_t st, const uint16_t* in, int64_t numel,
-                                bool weights_rule, uint64_t* sample, uint64_t* zero,
+                                int64_t zeros, bool weights_rule, uint64_t* sample, uint64_t* zero,
                                 int32_t* guess, int32_t* zero32);
 
 
@@ -2260,8 +2299,8 @@ extern "C" int zs_compress_retiled_fixed_gpu(void* stream, const uint16_t* d_inp
   const int64_t nrec = (int64_t)(M / 16) * (K / 64);
   if (nrec + 1 > INT32_MAX) return ZS_E_OVERFLOW;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(rfixed_kernel<false>, dim3(r_grid(nrec, 4)), dim3(256), 0, st, d_input, M,
-                     K, d_top_exponents, d_fixed, d_counts, d_tmp, nullptr, nullptr,
+  hipLaunchKernelGGL((rfixed_kernel<false, MatSrc>), dim3(r_grid(nrec, 4)), dim3(256), 0, st,
+                     MatSrc{d_input, K}, M, K, d_top_exponents, d_fixed, d_counts, d_tmp, nullptr, nullptr,
                      WindowCheck{});
   launch_rscan(st, d_counts, nrec, d_eoff, d_total);
   return status_of(hipGetLastError());
@@ -2279,14 +2318,18 @@ __global__ void zero_i32_kernel(int32_t* p, int64_t n) {
   if (i < n) p[i] = 0;
 }
 
-static int retiled_auto(void* stream, const uint16_t* d_input, int M, int K, int rule,
-                        const int32_t* d_guess, uint64_t* d_hist, int32_t* d_top, uint8_t* d_work,
-                        uint8_t* d_fixed, int32_t* d_counts, int32_t* d_eoff, int64_t* d_total,
-                        uint8_t* d_tmp) {
-  if (!shape_ok(M, K) || !d_input || !d_hist || !d_top || !d_work || !d_fixed || !d_counts ||
+// The one-pass encoder over the M x K matrix of `src`.  The guess is taken
+// from d_guess, or sampled from the n dense elements at `dense` (the matrix, or
+// the cache behind it, whose padding adds `zeros` elements).
+template <typename Src>
+static int retiled_auto(void* stream, const Src& src, const uint16_t* dense, int64_t n,
+                        int64_t zeros, int M, int K, int rule, const int32_t* d_guess,
+                        uint64_t* d_hist, int32_t* d_top, uint8_t* d_work, uint8_t* d_fixed,
+                        int32_t* d_counts, int32_t* d_eoff, int64_t* d_total, uint8_t* d_tmp) {
+  if (!shape_ok(M, K) || !dense || !d_hist || !d_top || !d_work || !d_fixed || !d_counts ||
       !d_eoff || !d_total || !d_tmp || (rule != ZS_WINDOW_KV && rule != ZS_WINDOW_WEIGHTS))
     return ZS_E_INVAL;
-  if ((reinterpret_cast<uintptr_t>(d_input) & 15) || (reinterpret_cast<uintptr_t>(d_fixed) & 15) ||
+  if ((reinterpret_cast<uintptr_t>(dense) & 15) || (reinterpret_cast<uintptr_t>(d_fixed) & 15) ||
       (reinterpret_cast<uintptr_t>(d_hist) & 7) || (reinterpret_cast<uintptr_t>(d_work) & 7))
     return ZS_E_INVAL;
   const int64_t nrec = (int64_t)(M / 16) * (K / 64);
@@ -2305,17 +2348,18 @@ static int retiled_auto(void* stream, const uint16_t* d_input, int M, int K, int
                        reinterpret_cast<int32_t*>(d_work), (int64_t)(kWorkArrive / 4 + 1));
     guess = const_cast<int32_t*>(d_guess);
   } else {
-    const hipError_t e = launch_window_sample(st, d_input, (int64_t)M * K, weights, sample, slices,
+    const hipError_t e = launch_window_sample(st, dense, n, zeros, weights, sample, slices,
                                               guess, arrive);
     if (e != hipSuccess) return status_of(e);
   }
   const int hist_grid = r_grid(nrec, 4);
-  hipLaunchKernelGGL(rfixed_kernel<true>, dim3(hist_grid), dim3(256), 0, st, d_input, M, K, guess,
+  hipLaunchKernelGGL((rfixed_kernel<true, Src>), dim3(hist_grid), dim3(256), 0, st, src, M, K, guess,
                      d_fixed, d_counts, d_tmp, slices, nullptr, WindowCheck{});
   // The window check, and a second encoding only when the window differs
   // from the guess (a small grid keeps the usual no-op launch cheap).
-  hipLaunchKernelGGL(rfixed_kernel<false>, dim3(std::min(r_grid(nrec, 4), device_cu_count() * 2)),
-                     dim3(256), 0, st, d_input, M, K, d_top, d_fixed, d_counts, d_tmp, nullptr,
+  hipLaunchKernelGGL((rfixed_kernel<false, Src>),
+                     dim3(std::min(r_grid(nrec, 4), device_cu_count() * 2)), dim3(256), 0, st, src,
+                     M, K, d_top, d_fixed, d_counts, d_tmp, nullptr,
                      nullptr, WindowCheck{slices, d_hist, d_top, guess, differs, weights ? 1 : 0});
   launch_rscan(st, d_counts, nrec, d_eoff, d_total, arrive);
   return status_of(hipGetLastError());
@@ -2325,7 +2369,7 @@ extern "C" int zs_compress_retiled_auto_gpu(void* stream, const uint16_t* d_inpu
                                             int rule, uint64_t* d_hist, int32_t* d_top,
                                             uint8_t* d_work, uint8_t* d_fixed, int32_t* d_counts,
                                             int32_t* d_eoff, int64_t* d_total, uint8_t* d_tmp) {
-  return retiled_auto(stream, d_input, M, K, rule, nullptr, d_hist, d_top, d_work, d_fixed,
+  return retiled_auto(stream, MatSrc{d_input, K}, d_input, (int64_t)M * K, 0, M, K, rule, nullptr, d_hist, d_top, d_work, d_fixed,
                       d_counts, d_eoff, d_total, d_tmp);
 }
 
@@ -2335,21 +2379,76 @@ extern "C" int zs_compress_retiled_guess_gpu(void* stream, const uint16_t* d_inp
                                              int32_t* d_counts, int32_t* d_eoff, int64_t* d_total,
                                              uint8_t* d_tmp) {
   if (!d_guess || d_guess == d_top) return ZS_E_INVAL;
-  return retiled_auto(stream, d_input, M, K, rule, d_guess, d_hist, d_top, d_work, d_fixed,
+  return retiled_auto(stream, MatSrc{d_input, K}, d_input, (int64_t)M * K, 0, M, K, rule, d_guess, d_hist, d_top, d_work, d_fixed,
                       d_counts, d_eoff, d_total, d_tmp);
+}
+
+// A cache [batch][tokens][heads][head_dim] as the matrix of its layout.
+static int kv_src(const uint16_t* x, int layout, int batch, int tokens, int heads, int head_dim,
+                  int group_rows, KvSrc* src, int* M) {
+  if (!x || batch <= 0 || tokens <= 0 || heads <= 0 || head_dim <= 0 || (head_dim % 64) ||
+      group_rows <= 0 || (group_rows % 16) ||
+      (layout != ZS_LAYOUT_HEAD_MAJOR && layout != ZS_LAYOUT_TOKEN_MAJOR))
+    return ZS_E_INVAL;
+  const bool hm = layout == ZS_LAYOUT_HEAD_MAJOR;
+  const int64_t valid = hm ? tokens : (int64_t)tokens * heads;
+  const int64_t rows = (int64_t)batch * (hm ? heads : 1) * group_rows;
+  if (group_rows < valid) return ZS_E_INVAL;
+  if (rows > INT32_MAX) return ZS_E_OVERFLOW;
+  auto fast = [](uint32_t d) {
+    return FastDiv{d, d == 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1) / d)};
+  };
+  const int64_t token = (int64_t)heads * head_dim;
+  *src = KvSrc{x, fast(group_rows / 16), fast(hm ? heads : 1), tokens * token, head_dim,
+               hm ? token : head_dim, (int)valid};
+  *M = (int)rows;
+  return ZS_OK;
+}
+
+extern "C" int zs_compress_retiled_kv_gpu(void* stream, const uint16_t* d_cache, int layout,
+                                          int batch, int tokens, int heads, int head_dim,
+                                          int group_rows, int rule, uint64_t* d_hist,
+                                          int32_t* d_top, uint8_t* d_work, uint8_t* d_fixed,
+                                          int32_t* d_counts, int32_t* d_eoff, int64_t* d_total,
+                                          uint8_t* d_tmp) {
+  KvSrc src;
+  int M;
+  const int c = kv_src(d_cache, layout, batch, tokens, heads, head_dim, group_rows, &src, &M);
+  if (c != ZS_OK) return c;
+  const int64_t n = (int64_t)batch * tokens * heads * head_dim;
+  return retiled_auto(stream, src, d_cache, n, (int64_t)M * head_dim - n, M, head_dim, rule,
+                      nullptr, d_hist, d_top, d_work, d_fixed, d_counts, d_eoff, d_total, d_tmp);
+}
+
+template <typename Src>
+static int retiled_exps(void* stream, const Src& src, const uint16_t* dense, int M, int K,
+                        const int32_t* d_top, const int32_t* d_eoff, const uint8_t* d_tmp,
+                        uint8_t* d_exps) {
+  if (!shape_ok(M, K) || !dense || !d_top || !d_eoff || !d_tmp || !d_exps) return ZS_E_INVAL;
+  if (reinterpret_cast<uintptr_t>(dense) & 15) return ZS_E_INVAL;
+  const int64_t nrec = (int64_t)(M / 16) * (K / 64);
+  hipLaunchKernelGGL(rcompact_kernel<Src>, dim3(r_grid((nrec + kCompactRecs - 1) / kCompactRecs, 4)),
+                     dim3(256), 0, (hipStream_t)stream, src, M, K, d_top, d_eoff, d_tmp, d_exps);
+  return status_of(hipGetLastError());
 }
 
 extern "C" int zs_compress_retiled_exps_gpu(void* stream, const uint16_t* d_input, int M, int K,
                                             const int32_t* d_top_exponents, const int32_t* d_eoff,
                                             const uint8_t* d_tmp, uint8_t* d_exps) {
-  if (!shape_ok(M, K) || !d_input || !d_top_exponents || !d_eoff || !d_tmp || !d_exps)
-    return ZS_E_INVAL;
-  if (reinterpret_cast<uintptr_t>(d_input) & 15) return ZS_E_INVAL;
-  const int64_t nrec = (int64_t)(M / 16) * (K / 64);
-  hipLaunchKernelGGL(rcompact_kernel, dim3(r_grid((nrec + kCompactRecs - 1) / kCompactRecs, 4)), dim3(256), 0,
-                     (hipStream_t)stream,
-                     d_input, M, K, d_top_exponents, d_eoff, d_tmp, d_exps);
-  return status_of(hipGetLastError());
+  return retiled_exps(stream, MatSrc{d_input, K}, d_input, M, K, d_top_exponents, d_eoff, d_tmp,
+                      d_exps);
+}
+
+extern "C" int zs_compress_retiled_kv_exps_gpu(void* stream, const uint16_t* d_cache, int layout,
+                                               int batch, int tokens, int heads, int head_dim,
+                                               int group_rows, const int32_t* d_top_exponents,
+                                               const int32_t* d_eoff, const uint8_t* d_tmp,
+                                               uint8_t* d_exps) {
+  KvSrc src;
+  int M;
+  const int c = kv_src(d_cache, layout, batch, tokens, heads, head_dim, group_rows, &src, &M);
+  if (c != ZS_OK) return c;
+  return retiled_exps(stream, src, d_cache, M, head_dim, d_top_exponents, d_eoff, d_tmp, d_exps);
 }
 
 static Streams canon_streams(const uint8_t* sm, const uint16_t* full, const uint64_t* b1,
