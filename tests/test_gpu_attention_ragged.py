@@ -69,3 +69,16 @@ def test_ragged_lengths_past_the_cache_are_clamped(torch_cuda):
             for s in ([600, 0, 77], [1 << 30, -5, 77])]
         torch.cuda.synchronize()
         assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("B,T,Hkv,H,ragged", [
+    (40, 600, 8, 16, False),    # 320 units: two shared splits, 640 of 768 places
+    (50, 1500, 8, 16, False),   # 400 units: one-wave items (a shared split fills half a round)
+    (50, 1500, 8, 16, True),
+    (97, 300, 8, 8, False),     # 776 units: just over one round of shared items
+    (3, 4000, 1, 8, False),     # three units: splits at their smallest
+])
+def test_automatic_splits_of_larger_grids(torch_cuda, B, T, Hkv, H, ragged):
+    lens = _lens(B, T, B) if ragged else None
+    _check(_run(torch_cuda, B, T, Hkv, H, seqlens=lens, splits=0, seed=B, retiled=True), lens,
+           exact=False)

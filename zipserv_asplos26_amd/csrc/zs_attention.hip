@@ -43,6 +43,9 @@ constexpr int kModeDense = 1;    // dense bf16 caches
 constexpr int kModeRetiled = 2;  // re-tiled records (zs_rdecode.hpp)
 constexpr int kModePaged = 3;    // dense bf16 caches in pages through a block table
 
+// Combine buffer of kWpi > 1: per wave, 32 O values + m + l per lane.
+constexpr int kCombineBytes = kItemWaves * 34 * 64 * 4;
+
 template <int kMode>
 struct AttnLds {
   // per-workgroup decode tables, then per-wave stages and the V tile
@@ -51,7 +54,11 @@ struct AttnLds {
                                                          : 0;
   static constexpr int kWave = (kMode == kModeCanon ? 2 * kStBytes
                                 : kMode == kModeRetiled ? 2 * kExpStage : 0) + kVBytes;
-  static constexpr int bytes(int waves) { return kTables + waves * kWave; }
+  // a workgroup's LDS; waves that share one item also merge their states there
+  static constexpr int bytes(int waves, bool shared) {
+    return kTables + waves * kWave < kCombineBytes && shared ? kCombineBytes
+                                                             : kTables + waves * kWave;
+  }
 };
 
 struct AttnParams {
@@ -78,6 +85,7 @@ struct AttnParams {
   const int32_t* seqlens;       // [B] or null
   int seqlen_k, batch, heads, heads_k, group, splits, chunk;
   int balanced;                 // splits follow the sequences' lengths (AttnSeq)
+  int shared;                   // a workgroup's waves share one item
   float scale_log2;             // softmax_scale * log2(e)
 };
 
@@ -192,27 +200,48 @@ __device__ __forceinline__ void build_e1(uint4* e1, int start_exp, int tid, int 
   }
 }
 
+// Max / sum over lanes l, l^16, l^32, l^48 (the four row groups), in every
+// lane: v_permlane16_swap of x with itself leaves rows (0, 0, 2, 2) and
+// (1, 1, 3, 3) of x, v_permlane32_swap rows (0, 1, 0, 1) and (2, 3, 2, 3) --
+// vector instructions instead of the LDS permutes that a shuffle compiles to
+// (token-major kernel 61.3 -> 56.9 us on a ragged batch of 201 MB, head-major
+// 81.5 -> 80.0 us on 398 MB).
+__device__ __forceinline__ void row_swap16(float x, float& a, float& b) {
+  const uint32_t u = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void row_swap32(float x, float& a, float& b) {
+  const uint32_t u = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
 __device__ __forceinline__ float wave_max16(float x) {
-  // max over lanes l, l^16, l^32, l^48 (the four row groups)
-  x = fmaxf(x, __shfl_xor(x, 16));
-  return fmaxf(x, __shfl_xor(x, 32));
+  float a, b;
+  row_swap16(x, a, b);
+  row_swap32(fmaxf(a, b), a, b);
+  return fmaxf(a, b);
 }
 __device__ __forceinline__ float wave_sum16(float x) {
-  x += __shfl_xor(x, 16);
-  return x + __shfl_xor(x, 32);
+  float a, b;
+  row_swap16(x, a, b);
+  row_swap32(a + b, a, b);
+  return a + b;
 }
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
-  const __bf16 ha = (__bf16)a, hb = (__bf16)b;
-  return (uint32_t)__builtin_bit_cast(unsigned short, ha) |
-         ((uint32_t)__builtin_bit_cast(unsigned short, hb) << 16);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
 
 // Per-wave attention state over one (batch, KV head, token range): the q^T
 // fragments (B operand, lane l -> head l%16 of the group, dims 32c +
 // 8*(l/16)..+7), the O^T accumulators (lane l: head l%16, dims 16*i +
-// 4*(l/16) + r of O[i]), the running max and sum (log2 domain), and the
-// current 16 tokens' scores S^T and softmax weights P^T (bf16 pairs).
+// 4*(l/16) + r of O[i]), the running max and this lane's share of the sum
+// (log2 domain), and the current 16 tokens' scores S^T and softmax weights P^T (bf16 pairs).
 struct AttnWave {
   bf16x8 Q[4];
   f32x4 O[8];
@@ -230,18 +259,24 @@ __device__ __forceinline__ void attn_k_step(AttnWave& a, int TY, u32x4 a0, u32x4
   a.S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a1), a.Q[2 * TY + 1], a.S, 0, 0, 0);
 }
 
-// Online softmax over the 16 tokens of S^T (log2 domain): this lane holds
-// tokens tb..tb+3 of head l%16; tokens >= t1 are masked.  Rescales O and
+// Online softmax over the 16 tokens of S^T from t on (log2 domain): this lane
+// holds tokens t + 4*(l/16) + 0..3 of head l%16; tokens >= t1 are masked --
+// kLast: behind a wave-uniform test, for only the range's last 16 tokens have
+// any (1.5% of the head-major kernel's time, but 2% the other way between the
+// token-major kernel's barriers).  Rescales O and
 // leaves the bf16 weights in pb0 / pb1 (the B operand P^T of the V steps).
-__device__ __forceinline__ void attn_softmax(AttnWave& a, int tb, int t1, float scale_log2) {
+template <bool kLast>
+__device__ __forceinline__ void attn_softmax(AttnWave& a, int t, int t1, float scale_log2) {
   float s[4];
-  float mx = -INFINITY;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    s[r] = (tb + r < t1) ? a.S[r] * scale_log2 : -INFINITY;
-    mx = fmaxf(mx, s[r]);
+  for (int r = 0; r < 4; ++r) s[r] = a.S[r] * scale_log2;
+  if (!kLast || t + 16 > t1) {
+    const int tb = t + 4 * (lane_id() >> 4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (tb + r >= t1) s[r] = -INFINITY;
   }
-  mx = wave_max16(mx);
+  const float mx = wave_max16(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
   const float m_new = fmaxf(a.m_run, mx);
   const float m_use = m_new == -INFINITY ? 0.f : m_new;
   const float alpha = __builtin_amdgcn_exp2f(a.m_run - m_use);
@@ -251,8 +286,7 @@ __device__ __forceinline__ void attn_softmax(AttnWave& a, int tb, int t1, float 
     pr[r] = __builtin_amdgcn_exp2f(s[r] - m_use);
     ps += pr[r];
   }
-  ps = wave_sum16(ps);
-  a.l_run = a.l_run * alpha + ps;
+  a.l_run = a.l_run * alpha + ps;  // this lane's tokens; summed over the lanes at the end
   if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) a.O[i] *= alpha;
@@ -287,9 +321,6 @@ __device__ __forceinline__ int kv_median(int rowbase, int med) {
   return ((rowbase >> 4) + med) & 3;
 }
 
-// Combine buffer of kWpi > 1: per wave, 32 O values + m + l per lane.
-constexpr int kCombineBytes = kItemWaves * 34 * 64 * 4;
-
 // kWpi = 1: the workgroup's kAttnWaves waves take one (batch, KV head,
 // split) item each.  kWpi = kItemWaves: its waves share one item, each a
 // contiguous 1/kWpi of the split's tokens, and merge their softmax states in
@@ -302,7 +333,9 @@ template <int kMode, int kWpi>
 __global__ __launch_bounds__((kWpi == 1 ? kAttnWaves : kWpi) * 64,
                              kMode == kModeRetiled ? 3 : 1) void attn_kernel(AttnParams p) {
   constexpr bool kDense = kMode == kModeDense || kMode == kModePaged;
-  extern __shared__ __attribute__((aligned(16))) uint8_t attn_smem[];
+  // (a static array: the offsets into it fold into the LDS instructions)
+  __shared__ __attribute__((aligned(16)))
+  uint8_t attn_smem[AttnLds<kMode>::bytes(kWpi == 1 ? kAttnWaves : kWpi, kWpi > 1)];
   DecodeTables& T = *reinterpret_cast<DecodeTables*>(attn_smem);
   RTables& RT = *reinterpret_cast<RTables*>(attn_smem);
   uint4* e1v = reinterpret_cast<uint4*>(
@@ -415,7 +448,7 @@ __global__ __launch_bounds__((kWpi == 1 ? kAttnWaves : kWpi) * 64,
   auto consume = [&](int TY, int med, u32x4 a0, u32x4 a1) {
     if (TY < 2) {
       attn_k_step(A, TY, a0, a1);
-      if (TY == 1) attn_softmax(A, t0 + 16 * med + 4 * (l >> 4), t1, p.scale_log2);
+      if (TY == 1) attn_softmax<true>(A, t0 + 16 * med, t1, p.scale_log2);
     } else {
       // V^T P^T for the 64 dims of this column tile, via the LDS transpose
       *reinterpret_cast<u32x4*>(vbuf + vwr) = a0;
@@ -521,11 +554,8 @@ __global__ __launch_bounds__((kWpi == 1 ? kAttnWaves : kWpi) * 64,
     r_stage(NXT, RN, MN);                                                               \
     ZR_ISSUE(ZR_CLAMP((J) + 4, I), I, RC, MC);                                          \
     u32x4 a0_, a1_;                                                                     \
-    if (r_staged(cm_))                                                                  \
-      r_decode(RT, (I) < 2 ? kex : vex, cs_.r, (const uint8_t*)(CUR), cm_.rel, a0_, a1_);   \
-    else                                                                                \
-      r_decode(RT, (I) < 2 ? kex : vex, cs_.r, ((I) < 2 ? p.kexp : p.vexp) + cm_.e0,    \
-               0, a0_, a1_);                                                            \
+    r_decode_staged(RT, (I) < 2 ? kex : vex, cs_, cm_, CUR, (I) < 2 ? p.kexp : p.vexp, \
+                    a0_, a1_);                                                         \
     consume((I), (c0 + (J)) >> 2, a0_, a1_);                                            \
   }
         if (c0 > 0) {  // chunk 0's first steps were issued at start-up
@@ -603,6 +633,7 @@ __global__ __launch_bounds__((kWpi == 1 ? kAttnWaves : kWpi) * 64,
     }
   }
 
+  A.l_run = wave_sum16(A.l_run);
   if constexpr (kWpi > 1) {
     // Merge the waves' softmax states (log2 domain) into wave 0; the decode
     // tables are dead by now, their LDS holds the states.
@@ -840,11 +871,8 @@ __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(
     r_stage(NXT, RN, MN);                                                                  \
     ZT_ISSUE(ZT_CLAMP((J) + D, I), I, RC, MC);                                             \
     u32x4 a0_, a1_;                                                                        \
-    if (r_staged(cm_))                                                                     \
-      r_decode(RT, (I) < 2 ? kex : vex, cs_.r, (const uint8_t*)(CUR), cm_.rel, a0_, a1_);  \
-    else                                                                                   \
-      r_decode(RT, (I) < 2 ? kex : vex, cs_.r, ((I) < 2 ? p.kexp : p.vexp) + cm_.e0, 0,    \
-               a0_, a1_);                                                                  \
+    r_decode_staged(RT, (I) < 2 ? kex : vex, cs_, cm_, CUR, (I) < 2 ? p.kexp : p.vexp, \
+                    a0_, a1_);                                                         \
     uint8_t* xt_ = xch + (I) * kTmPhase;                                                   \
     *reinterpret_cast<u32x4*>(xt_ + xwr) = a0_;                                            \
     *reinterpret_cast<u32x4*>(xt_ + xwr + 64) = a1_;                                       \
@@ -855,7 +883,7 @@ __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(
     const u32x4 k0_ = *reinterpret_cast<const u32x4*>(xt_ + krd);                          \
     const u32x4 k1_ = *reinterpret_cast<const u32x4*>(xt_ + krd + 64);                     \
     attn_k_step(A, (I), k0_, k1_);                                                         \
-    if ((I) == 1) attn_softmax(A, t0 + 16 * ((c0 + (J)) >> 2) + 4 * (l >> 4), t1, p.scale_log2); \
+    if ((I) == 1) attn_softmax<false>(A, t0 + 16 * ((c0 + (J)) >> 2), t1, p.scale_log2); \
   }
 #define ZT_STEP(J, I, CUR, NXT, RC, MC, RN, MN)                                            \
   {                                                                                        \
@@ -864,11 +892,8 @@ __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(
     r_stage(NXT, RN, MN);                                                                  \
     ZT_ISSUE(ZT_CLAMP((J) + D, I), I, RC, MC);                                             \
     u32x4 a0_, a1_;                                                                        \
-    if (r_staged(cm_))                                                                     \
-      r_decode(RT, (I) < 2 ? kex : vex, cs_.r, (const uint8_t*)(CUR), cm_.rel, a0_, a1_);  \
-    else                                                                                   \
-      r_decode(RT, (I) < 2 ? kex : vex, cs_.r, ((I) < 2 ? p.kexp : p.vexp) + cm_.e0, 0,    \
-               a0_, a1_);                                                                  \
+    r_decode_staged(RT, (I) < 2 ? kex : vex, cs_, cm_, CUR, (I) < 2 ? p.kexp : p.vexp, \
+                    a0_, a1_);                                                         \
     uint8_t* xt_ = xch + ((I) & 1) * kTmPhase;                                             \
     *reinterpret_cast<u32x4*>(xt_ + xwr) = a0_;                                            \
     *reinterpret_cast<u32x4*>(xt_ + xwr + 64) = a1_;                                       \
@@ -878,7 +903,7 @@ __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(
       const u32x4 k1_ = *reinterpret_cast<const u32x4*>(xt_ + krd + 64);                   \
       attn_k_step(A, (I), k0_, k1_);                                                       \
       if ((I) == 1)                                                                        \
-        attn_softmax(A, t0 + 16 * ((c0 + (J)) >> 2) + 4 * (l >> 4), t1, p.scale_log2);    \
+        attn_softmax<false>(A, t0 + 16 * ((c0 + (J)) >> 2), t1, p.scale_log2);    \
     } else {                                                                               \
       attn_v_step(A, (I), xt_ + vtr);                                                      \
     }                                                                                      \
@@ -926,6 +951,7 @@ __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(
   }
 
   // Results, as attn_kernel: lane l holds head h * group + l%16.
+  A.l_run = wave_sum16(A.l_run);
   const int head = h * p.group + g;
   const bool own = g < p.group;
   const int d0 = 4 * (l >> 4);
@@ -1069,8 +1095,10 @@ static hipError_t launch_combine(hipStream_t st, const AttnParams& p) {
   return hipGetLastError();
 }
 
-// Workgroups of four waves per item take grids of fewer than this many items.
+// Workgroups of four waves per item take grids of fewer than this many items,
+// unless attn_split_retiled says otherwise.
 constexpr int kSharedItemsBelow = 2048;
+int device_cu_count();  // zs_gemm.hip
 
 static int attn_auto_splits(int batch, int heads_k, int seqlen_k, bool compressed) {
   // One wave per item: about 2048 waves, at least 256 tokens per split.
@@ -1089,6 +1117,52 @@ static int attn_auto_splits(int batch, int heads_k, int seqlen_k, bool compresse
   return std::min(max_shared, std::max(1, (items + units - 1) / units));
 }
 
+// Splits of the re-tiled mode, and whether a workgroup's four waves share one
+// item.  Three of its workgroups fit a CU (45 KB of LDS, 128 VGPRs), and one
+// full round of them is what is fast: 768 shared items, or 3072 of one wave
+// (the merge of four waves in LDS saves three quarters of the partial results,
+// 2-8% at equal rounds).  Grids of 2048 one-wave items, two thirds of a round,
+// or somewhat over one lose up to 20%: B = 24, T = 6000 110 -> 90.5 us, B = 8,
+// T = 8k 50.0 -> 43.8, T = 16k 90.0 -> 80.6, B = 16, T = 4k 50.0 -> 43.9, B =
+// 3, T = 10000 32.0 -> 25.7 (64 / 8 heads; every count of 384..6144 items,
+// both orders).  Past 64 splits a (batch, head)'s merge costs what the fuller
+// round gains (B = 1, T = 32k: 96 splits 30.7, 64 splits 29.7 us).
+struct AttnSplit {
+  int splits;
+  bool shared;
+};
+static AttnSplit attn_split_retiled(int batch, int heads_k, int seqlen_k) {
+  const int64_t units = std::max<int64_t>(1, (int64_t)batch * heads_k);
+  const int64_t slots = 3 * (int64_t)device_cu_count();
+  auto pick = [&](int64_t slots, int min_tokens, int64_t most) {
+    const int64_t fit = (seqlen_k + min_tokens - 1) / min_tokens;
+    return std::max<int64_t>(1, std::min({slots / units, fit, most}));
+  };
+  // the share of its rounds that a grid fills
+  auto filled = [](int64_t items, int64_t slots) {
+    return (double)items / ((items + slots - 1) / slots * slots);
+  };
+  const int64_t sh = pick(slots, 128, 64), one = pick(slots * kAttnWaves, 256, INT32_MAX);
+  const double fs = filled(sh * units, slots), fo = filled(one * units, slots * kAttnWaves);
+  if (fs >= 0.9 * fo) return {(int)sh, true};
+  return {(int)one, false};
+}
+
+// Splits of the canonical mode (two workgroups a CU).
+static AttnSplit attn_split_canonical(int batch, int heads_k, int seqlen_k) {
+  const int s = attn_auto_splits(batch, heads_k, seqlen_k, true);
+  return {s, (int64_t)s * batch * heads_k < kSharedItemsBelow};
+}
+
+// Splits of the dense modes: on large grids the re-tiled mode's, so that the
+// two walk the same pieces, else attn_auto_splits.
+static AttnSplit attn_split_dense(int batch, int heads_k, int seqlen_k) {
+  const int s = attn_auto_splits(batch, heads_k, seqlen_k, false);
+  if ((int64_t)s * batch * heads_k >= kSharedItemsBelow)
+    return attn_split_retiled(batch, heads_k, seqlen_k);
+  return {s, true};
+}
+
 // Tokens per split: a multiple of 16 (one median, one record band), so that
 // every wave's range starts on a band of every layout.
 static int attn_chunk(int seqlen_k, int splits) {
@@ -1100,6 +1174,17 @@ static int attn_chunk(int seqlen_k, int splits) {
 // library's choice, there are lengths to follow and more than one split.
 static int attn_balanced(const AttnParams& p, int num_splits) {
   return num_splits == 0 && p.seqlens && p.splits > 1 && p.batch > 1;
+}
+
+// The splits of a call: num_splits of them, or this library's choice `own`.
+static void attn_set_splits(AttnParams& p, int num_splits, AttnSplit own) {
+  const int steps = std::max(1, (p.seqlen_k + 15) / 16);
+  p.splits = std::max(1, std::min(num_splits > 0 ? num_splits : own.splits, steps));
+  p.chunk = attn_chunk(std::max(p.seqlen_k, 1), p.splits);
+  p.balanced = attn_balanced(p, num_splits);
+  p.shared = p.chunk > 64 &&
+             (num_splits > 0 ? (int64_t)p.batch * p.heads_k * p.splits < kSharedItemsBelow
+                             : own.shared);
 }
 
 static size_t attn_ws_bytes(int batch, int heads, int splits) {
@@ -1115,15 +1200,13 @@ static int attn_launch(hipStream_t st, AttnParams& p, void* workspace, size_t ws
     p.ws_ml = p.ws_o + (size_t)p.batch * p.heads * p.splits * kHeadDim;
   }
   const int items = p.batch * p.heads_k * p.splits;
-  if (items < kSharedItemsBelow && p.chunk > 64) {
-    // small grid: four waves per item
-    const size_t lds = std::max<size_t>(AttnLds<kMode>::bytes(kItemWaves), kCombineBytes);
-    hipLaunchKernelGGL((attn_kernel<kMode, kItemWaves>), dim3(items), dim3(kItemWaves * 64), lds,
-                       st, p);
+  if (p.shared) {
+    // four waves per item
+    hipLaunchKernelGGL((attn_kernel<kMode, kItemWaves>), dim3(items), dim3(kItemWaves * 64), 0, st,
+                       p);
   } else {
     const int grid = (items + kAttnWaves - 1) / kAttnWaves;
-    const size_t lds = AttnLds<kMode>::bytes(kAttnWaves);
-    hipLaunchKernelGGL((attn_kernel<kMode, 1>), dim3(grid), dim3(kAttnWaves * 64), lds, st, p);
+    hipLaunchKernelGGL((attn_kernel<kMode, 1>), dim3(grid), dim3(kAttnWaves * 64), 0, st, p);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
@@ -1162,8 +1245,6 @@ static size_t staging_bytes(int layout, int rows, int cols) {
   if (layout != ZS_LAYOUT_TOKEN_MAJOR) return 0;
   return ((size_t)rows * cols * 2 + 255) / 256 * 256;
 }
-
-int device_cu_count();  // zs_gemm.hip
 
 // Fused token-major attention (attn_tm_kernel) takes re-tiled caches with
 // kTmHeads KV heads; other token-major caches run staged.
@@ -1247,12 +1328,13 @@ extern "C" size_t zs_decode_attention_workspace_bytes(int batch, int num_heads, 
                                                       int seqlen_k, int num_splits) {
   if (batch <= 0 || num_heads <= 0 || head_dim != kHeadDim || seqlen_k < 0) return 0;
   // num_splits == 0 asks for the automatic choice, which never exceeds
-  // min(ceil(T/128), ceil(2048/batch)) splits, or for fused token-major
-  // caches min(ceil(T/16), ceil(kTmItems/batch)).
+  // min(ceil(T/128), max(ceil(2048/batch), 12 per CU / batch)) splits, or for
+  // fused token-major caches min(ceil(T/16), ceil(kTmItems/batch)).
   const int splits =
       num_splits > 0
           ? num_splits
-          : std::max(std::min(std::max(1, (seqlen_k + 127) / 128), (2048 + batch - 1) / batch),
+          : std::max(std::min(std::max(1, (seqlen_k + 127) / 128),
+                              (std::max(2048, 12 * device_cu_count()) + batch - 1) / batch),
                      std::min(std::max(1, (seqlen_k + 15) / 16), (kTmItems + batch - 1) / batch));
   return attn_ws_bytes(batch, num_heads, splits);
 }
@@ -1314,11 +1396,10 @@ extern "C" int zs_decode_attention(void* stream, const uint16_t* q, const zs_kv_
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
-  p.splits = num_splits > 0 ? num_splits : attn_auto_splits(batch, num_heads_k, seqlen_k,
-                                                                 k->layout != ZS_LAYOUT_TOKEN_MAJOR);
-  p.splits = std::max(1, std::min(p.splits, std::max(1, (seqlen_k + 15) / 16)));
-  p.chunk = attn_chunk(std::max(seqlen_k, 1), p.splits);
-  p.balanced = attn_balanced(p, num_splits);
+  attn_set_splits(p, num_splits,
+                  k->layout != ZS_LAYOUT_TOKEN_MAJOR
+                      ? attn_split_canonical(batch, num_heads_k, seqlen_k)
+                      : attn_split_dense(batch, num_heads_k, seqlen_k));
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   if (k->layout == ZS_LAYOUT_TOKEN_MAJOR) {
     const size_t sk = staging_bytes(k->layout, k->rows, k->cols);
@@ -1396,11 +1477,11 @@ extern "C" int zs_decode_attention_retiled(void* stream, const uint16_t* q,
     p.balanced = attn_balanced(p, num_splits);
     return attn_tm_launch((hipStream_t)stream, p, workspace, workspace_bytes);
   }
-  p.splits = num_splits > 0 ? num_splits : attn_auto_splits(batch, num_heads_k, seqlen_k,
-                                                                 k->layout != ZS_LAYOUT_TOKEN_MAJOR);
-  p.splits = std::max(1, std::min(p.splits, std::max(1, (seqlen_k + 15) / 16)));
-  p.chunk = attn_chunk(std::max(seqlen_k, 1), p.splits);
-  p.balanced = attn_balanced(p, num_splits);
+  // (a staged cache runs in the dense mode, with its splits)
+  attn_set_splits(p, num_splits,
+                  k->layout != ZS_LAYOUT_TOKEN_MAJOR
+                      ? attn_split_retiled(batch, num_heads_k, seqlen_k)
+                      : attn_split_dense(batch, num_heads_k, seqlen_k));
   if (k->layout == ZS_LAYOUT_TOKEN_MAJOR) {
     const size_t sk = staging_bytes(k->layout, k->rows, k->cols);
     const size_t sv = staging_bytes(v->layout, v->rows, v->cols);
@@ -1446,10 +1527,7 @@ extern "C" int zs_decode_attention_dense(void* stream, const uint16_t* q, const 
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
-  p.splits = num_splits > 0 ? num_splits : attn_auto_splits(batch, num_heads_k, seqlen_k, false);
-  p.splits = std::max(1, std::min(p.splits, std::max(1, (seqlen_k + 15) / 16)));
-  p.chunk = attn_chunk(std::max(seqlen_k, 1), p.splits);
-  p.balanced = attn_balanced(p, num_splits);
+  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k));
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   return attn_launch<kModeDense>((hipStream_t)stream, p, workspace, workspace_bytes);
 }
@@ -1483,10 +1561,7 @@ extern "C" int zs_decode_attention_dense_paged(
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
-  p.splits = num_splits > 0 ? num_splits : attn_auto_splits(batch, num_heads_k, seqlen_k, false);
-  p.splits = std::max(1, std::min(p.splits, std::max(1, (seqlen_k + 15) / 16)));
-  p.chunk = attn_chunk(std::max(seqlen_k, 1), p.splits);
-  p.balanced = attn_balanced(p, num_splits);
+  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k));
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   return attn_launch<kModePaged>((hipStream_t)stream, p, workspace, workspace_bytes);
 }
