@@ -662,46 +662,13 @@ def bench_kv(torch, zs, dev, gen):
 
 
 def kernel_name(N, M, split_k, K):
-    """Kernel that zs_retiled_mm launches for batch N (mirrors its dispatch):
-    N <= 16 -> rgemm_kernel<F, 1, W, D, XD> (F bands per wave: 2 when N > 8
-    and M/16 >= 384, else 1; one 16-column block; W = 4 waves when M/16 >= 640
-    (N > 1) or M/16 >= 896 (N = 1), else 8; records D = 4 tiles ahead with one
-    band per wave, 3
-    with two; X staged through LDS in XD-row loads: 1 for N <= 2, 2 for
-    N <= 4, 4 for N <= 8, none (0) above); N > 16 ->
-    rgemm_wide_kernel<NB, 4, PH, 2> with NB = 2, 4 or 8
-    column blocks, 4 row bands, 4 K phases when M/64 * split_k <= the CU
-    count (2 otherwise), records 2 steps ahead; on grids of >= 160 128-row
-    workgroups rgemm_wide2_kernel<NB, 8, 2> (two bands per wave) instead,
-    for N > 64 at any split-K and for 16 < N <= 64 at split-K 1 or 2;
-    4 <= N <= 16 on grids of M/64 * split_k >= 7/8 of the CU count ->
-    rgemm_wide_kernel<1, 4, PH, 2>; NB = 8 outside the two-band case takes 3
-    K phases when the split-K slice has >= 32 K tiles."""
-    import torch
-    nb = (N + 15) // 16
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    """Kernel that zs_retiled_mm launches for batch N (zs_retiled_mm_kernel),
+    or for split_k == 0 zs_retiled_mm_streamk."""
+    import zipserv_asplos26_amd as zs
     if split_k == 0:  # stream-K schedule (narrow batches)
         xd = 1 if N <= 2 else (2 if N <= 4 else (4 if N <= 8 else 0))
         return f"zs::rgemm_sk_kernel<4, {xd}>"
-    if nb <= 1 and N >= 4 and (M // 64) * split_k * 8 >= cus * 7:
-        ph = 4 if (M // 64) * split_k <= cus else 2
-        return f"zs::rgemm_wide_kernel<1, 4, {ph}, 2>"
-    if nb <= 1:
-        waves = 4 if M // 16 >= (640 if N > 1 else 896) else 8
-        f = 2 if (N > 8 and M // 16 >= 384) else 1
-        xd = 1 if N <= 2 else (2 if N <= 4 else (4 if N <= 8 else 0))
-        return f"zs::rgemm_kernel<{f}, 1, {waves}, {4 if f == 1 else 3}, {xd}>"
-    nb = 2 if nb <= 2 else (4 if nb <= 4 else 8)
-    if nb == 2 and M % 128 == 0 and split_k <= 2 and (M // 128) * split_k >= 160:
-        return "zs::rgemm_wide2_kernel<2, 8, 2>"
-    if nb == 8 and M % 128 == 0 and (M // 128) * split_k * ((N + 127) // 128) >= 160:
-        return "zs::rgemm_wide2_kernel<8, 8, 2>"
-    if nb == 4 and M % 128 == 0 and split_k <= 2 and (M // 128) * split_k >= 160:
-        return "zs::rgemm_wide2_kernel<4, 8, 2>"
-    ph = 4 if (nb <= 4 and (M // 64) * split_k <= cus) else 2
-    if nb == 8 and ((K // 64) - 1) // split_k + 1 >= 32:
-        ph = 3
-    return f"zs::rgemm_wide_kernel<{nb}, 4, {ph}, 2>"
+    return zs.lib().zs_retiled_mm_kernel(M, N, K, split_k).decode()
 
 
 def compress_kernel_seconds(torch, zs, x, window="kv", reps=3):

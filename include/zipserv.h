@@ -285,6 +285,10 @@ int zs_retiled_decompress(void* stream, const uint8_t* d_fixed, const uint8_t* d
 int zs_retiled_mm(void* stream, const uint8_t* d_fixed, const uint8_t* d_exps,
                   const int32_t* d_eoff, uint8_t start_exp, const uint16_t* B, uint16_t* C, int M,
                   int N, int K, uint16_t* Reduction_Workspace, int Split_K);
+/* Name of the GEMM kernel that zs_retiled_mm, _fused and _fused_noalloc launch
+ * for this shape on the current device (as a profiler shows it), NULL for a
+ * shape they refuse.  No counterpart in the reference. */
+const char* zs_retiled_mm_kernel(int M, int N, int K, int split_k);
 /* zs_retiled_mm with the split-K reduction inside the GEMM kernel (no
  * counterpart in the reference, whose split-K always runs
  * SplitK_Reduction, build/L_API.cuh:19-37): every workgroup stores its bf16

@@ -79,6 +79,7 @@ SIGNATURES = {
     "zs_retiled_decompress": (C.c_int, [_p, _p, _p, _p, C.c_uint8, _p, C.c_int, C.c_int]),
     "zs_retiled_mm": (C.c_int, [_p, _p, _p, _p, C.c_uint8, _p, _p, C.c_int, C.c_int, C.c_int,
                                 _p, C.c_int]),
+    "zs_retiled_mm_kernel": (C.c_char_p, [C.c_int] * 4),
     "zs_retiled_mm_counters": (C.c_int64, [C.c_int, C.c_int]),
     "zs_retiled_mm_streamk_workspace_bytes": (C.c_int64, [C.c_int, C.c_int, C.c_int]),
     "zs_retiled_mm_streamk": (C.c_int, [_p, _p, _p, _p, C.c_uint8, _p, _p, C.c_int, C.c_int,

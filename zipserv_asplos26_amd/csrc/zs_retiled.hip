@@ -2516,8 +2516,131 @@ extern "C" int zs_retiled_decompress(void* stream, const uint8_t* d_fixed, const
   return status_of(hipGetLastError());
 }
 
-// Split-K partial sums go to ws; with `counters` the GEMM kernel itself adds
-// them (last workgroup per tile), without it rsplitk_reduce_kernel does.
+// ---------------------------------------------------------------------------
+// Which ZipGEMM kernel a call runs.
+// ---------------------------------------------------------------------------
+namespace zs {
+
+using MmLaunch = hipError_t (*)(hipStream_t, const uint8_t*, const uint8_t*, const int32_t*, int,
+                                const uint16_t*, uint16_t*, int, int, int, int, int, SplitFix);
+
+struct MmKernel {
+  const char* name;
+  MmLaunch launch;
+  // N > 16: 16-column blocks and rows of a workgroup, workgroups that fit a CU
+  int nb, rows, per_cu, min_kt;
+  // and its time in us: start + round per round of the grid, load per K tile of
+  // the workgroups that the busiest CU gets, mean per K tile of the mean over
+  // the CUs, alone per K tile where two fit a CU and it gets one
+  // and its time in us: start, round per round of the grid, group per
+  // workgroup that the busiest CU gets, load per K tile of those, mean per K tile
+  // of the mean over the CUs, alone per K tile where two fit a CU and it gets one
+  float start, round, group, load, mean, alone;
+};
+
+// Wide kernels (N > 16).  The grid decides as much as the kernel: a split-K
+// slice of 4096 rows is 64 workgroups of 64 rows, a quarter of the chip, so
+// there narrower column blocks win that decode the records again in other
+// workgroups (4096 x 14336, N = 100: one slice 94.7 -> 55.7 us, two slices 54.9
+// -> 39.2; 2048 x 14336, N = 128: 96.4 -> 53.4); with 257..768 workgroups of 64
+// rows two of them a CU beat one of 128 rows (28672 x 8192, N = 24: 73.8 ->
+// 64.8; 20480 x 4096, N = 40: 44.7 -> 38.7), past that 128 rows win; and where a
+// grid falls just over a round, smaller column blocks fill it better (20480 x
+// 4096, N = 160: 101.4 -> 76.4).  So the kernel with the smallest modelled time
+// is taken.  The model's constants are a least-squares fit of relative error
+// over 915 (M, K, N = 17..500, split-K 1 / 2 / 4) points, every kernel timed at
+// each; its choice is on average 0.8% (at most 17%) over the fastest kernel, the
+// thresholds on M, N and split-K that it replaced 12.5% (at most 89%).  The
+// 128-row kernels of 2 and 4 blocks count 4% more than their fit, since in a near
+// tie the smaller tiles lose less, and three K phases take slices of >= 24 K
+// tiles (on 16 the uneven phases cost up to 6%).
+#define ZS_MM_WIDE(NB, PH) "zs::rgemm_wide_kernel<" #NB ", 4, " #PH ", 2>", launch_rwide<NB, 4, PH>, NB, 64
+#define ZS_MM_WIDE2(NB) "zs::rgemm_wide2_kernel<" #NB ", 8, 2>", launch_rwide2<NB, 8, 2>, NB, 128
+static_assert(kWideDepth == 2, "records ahead in the names");
+static const MmKernel kWideKernels[] = {
+    {ZS_MM_WIDE(1, 4), 1, 0, 2.706f, 1.935f, 0.000f, 0.164f, 0.036f, 0.000f},
+    {ZS_MM_WIDE(2, 4), 1, 0, 1.517f, 3.815f, 0.000f, 0.189f, 0.057f, 0.000f},
+    {ZS_MM_WIDE(3, 4), 1, 0, 1.546f, 4.558f, 0.000f, 0.207f, 0.061f, 0.000f},
+    {ZS_MM_WIDE(4, 4), 1, 0, 1.310f, 4.956f, 0.000f, 0.237f, 0.058f, 0.000f},
+    {ZS_MM_WIDE(2, 2), 2, 0, 1.592f, 2.359f, 0.663f, 0.183f, 0.061f, 0.102f},
+    {ZS_MM_WIDE(4, 2), 2, 0, 1.643f, 1.624f, 1.794f, 0.226f, 0.067f, 0.095f},
+    {ZS_MM_WIDE(8, 3), 1, 24, 1.452f, 6.028f, 0.000f, 0.374f, 0.068f, 0.000f},
+    {ZS_MM_WIDE(8, 2), 1, 0, 0.919f, 5.898f, 0.000f, 0.419f, 0.055f, 0.000f},
+    {ZS_MM_WIDE2(2), 2, 0, 1.404f, 2.531f, 1.904f, 0.366f, 0.099f, 0.145f},
+    {ZS_MM_WIDE2(4), 2, 0, 0.057f, 4.810f, 2.855f, 0.441f, 0.096f, 0.157f},
+    {ZS_MM_WIDE2(8), 1, 0, 0.998f, 8.192f, 0.000f, 0.669f, 0.089f, 0.000f},
+};
+
+constexpr int kMaxGridZ = 65535;  // column blocks of a launch
+
+static float mm_time(const MmKernel& k, int M, int N, int kt, int split_k, int64_t cus) {
+  const int64_t grid = (int64_t)(M / k.rows) * split_k * (((N + 15) / 16 + k.nb - 1) / k.nb);
+  const int64_t load = (grid + cus - 1) / cus;
+  const int64_t rounds = (grid + cus * k.per_cu - 1) / (cus * k.per_cu);
+  return k.start + k.round * rounds + k.group * load +
+         (k.load * load + k.mean * grid / cus + (load == 1 ? k.alone : 0.f)) * kt;
+}
+
+// Narrow kernels (N <= 16) of F bands per wave and W waves, records D tiles
+// ahead; the launch picks how X is staged from N, [i] names the choice.
+#define ZS_MM_NARROW(F, W, D)                                                              \
+  {{"zs::rgemm_kernel<" #F ", 1, " #W ", " #D ", 0>", launch_rgemm<F, 1, W>},              \
+   {"zs::rgemm_kernel<" #F ", 1, " #W ", " #D ", 1>", launch_rgemm<F, 1, W>},              \
+   {"zs::rgemm_kernel<" #F ", 1, " #W ", " #D ", 2>", launch_rgemm<F, 1, W>},              \
+   {"zs::rgemm_kernel<" #F ", 1, " #W ", " #D ", 4>", launch_rgemm<F, 1, W>}}
+static const MmKernel kNarrow14[4] = ZS_MM_NARROW(1, 4, 4), kNarrow18[4] = ZS_MM_NARROW(1, 8, 4),
+                      kNarrow24[4] = ZS_MM_NARROW(2, 4, 3), kNarrow28[4] = ZS_MM_NARROW(2, 8, 3);
+static const MmKernel kOneBlock4 = kWideKernels[0],
+                      kOneBlock2 = {"zs::rgemm_wide_kernel<1, 4, 2, 2>", launch_rwide<1, 4, 2>};
+
+static const MmKernel& mm_kernel(int M, int N, int K, int split_k) {
+  const int kt = (K / 64 - 1) / split_k + 1;
+  const int64_t cus = device_cu_count();
+  if (N > 16) {
+    const MmKernel* best = nullptr;
+    float least = 0.f;
+    for (const MmKernel& k : kWideKernels) {
+      if (M % k.rows || kt < k.min_kt || (k.nb < 8 && (N - 1) / (16 * k.nb) >= kMaxGridZ)) continue;
+      const float t = mm_time(k, M, N, kt, split_k, cus);
+      if (!best || t < least) best = &k, least = t;
+    }
+    return *best;
+  }
+  // One 16-column block: 64-row workgroups, four K phases where one round of
+  // them fits, two otherwise, from 4 <= N on grids of 7/8 of one per CU (each
+  // X tile crosses L2 once per four bands: 8-24% faster than one band per
+  // workgroup at N = 8 / 16 on such grids), and on 5/8 of one per CU for N > 8
+  // or slices of up to 64 K tiles (6144 x 4096, two slices: 18.6 -> 13.1 us at N =
+  // 16, 14.8 -> 13.0 at 8; 10240 x 8192, N = 16: 35.0 -> 31.8; not 128 of them:
+  // 8192 x 28672, N = 16 64.4 -> 98.6); short slices at any N, where a band's
+  // workgroup is mostly its start-up and, split, its arrival (10240 x 4096, N =
+  // 1, four slices: 1.78x; 16384 x 512, N = 3: 1.9-2.3x; one slice of 32 K tiles
+  // of 20480 rows at N = 1 is 18% slower so).
+  const int64_t wide = (int64_t)(M / 64) * split_k;
+  const bool full = wide >= cus, most = wide * 8 >= cus * 5;
+  if ((N >= 4 && wide * 8 >= cus * 7) || (most && (N > 8 || (N > 4 && kt <= 64) || kt <= 16)) ||
+      (full && split_k > 1 && kt <= 36))
+    return wide <= cus ? kOneBlock4 : kOneBlock2;
+  // Otherwise workgroups of 8 K phases over one band, or two bands for N > 8
+  // once the grid keeps at least 192 workgroups (half the X bytes per record,
+  // the cost that grows with N).  Workgroups of 4 waves (16 per CU, twice the
+  // K tiles per wave) instead of 8 for N > 1 on >= 640 bands (1-5 us faster at
+  // N = 8 / 16 on 10240, 14336 and 28672 rows, slower on smaller grids), for N
+  // = 1 on >= 896 bands (14336 rows: 21.9 -> 19.6 us; 10240 rows are 0.6 us
+  // slower with 4 waves), and on > 512 of them for slices of up to 16 K tiles.
+  const bool w4 = M / 16 >= (N > 1 ? 640 : 896) || (kt <= 16 && (int64_t)(M / 16) * split_k > 512);
+  const int xd = N <= 2 ? 1 : N <= 4 ? 2 : N <= 8 ? 3 : 0;
+  if (N > 8 && (int64_t)(M / 16) * split_k >= 384) return w4 ? kNarrow24[xd] : kNarrow28[xd];
+  return w4 ? kNarrow14[xd] : kNarrow18[xd];
+}
+
+}  // namespace zs
+
+extern "C" const char* zs_retiled_mm_kernel(int M, int N, int K, int split_k) {
+  if (!shape_ok(M, K) || N <= 0 || split_k < 1 || split_k > K / 64) return nullptr;
+  return mm_kernel(M, N, K, split_k).name;
+}
+
 // Argument checks of retiled_mm that do not depend on the split-K buffers.
 static int retiled_mm_args(const uint8_t* d_fixed, const uint8_t* d_exps, const int32_t* d_eoff,
                            const uint16_t* B, const uint16_t* C, int M, int N, int K,
@@ -2534,6 +2657,8 @@ static int retiled_mm_args(const uint8_t* d_fixed, const uint8_t* d_exps, const 
   return ZS_OK;
 }
 
+// Split-K partial sums go to ws; with `counters` the GEMM kernel itself adds
+// them (last workgroup per tile), without it rsplitk_reduce_kernel does.
 static int retiled_mm(void* stream, const uint8_t* d_fixed, const uint8_t* d_exps,
                       const int32_t* d_eoff, uint8_t start_exp, const uint16_t* B, uint16_t* C,
                       int M, int N, int K, uint16_t* ws, int split_k, int32_t* counters) {
@@ -2556,74 +2681,12 @@ static int retiled_mm(void* stream, const uint8_t* d_fixed, const uint8_t* d_exp
     return ZS_OK;
   }
   hipStream_t st = (hipStream_t)stream;
-  const int se = (int)start_exp;
-  hipError_t e;
   const int kb_per_split = (KT - 1) / split_k + 1;
   uint16_t* out = split_k == 1 ? C : ws;
   const SplitFix fx{C, split_k > 1 ? counters : nullptr, split_k};
-  const int nb = (N + 15) / 16;
-  // N > 16: 64-row workgroups sharing each X tile through LDS; four K phases
-  // per workgroup (16 waves, one workgroup per CU) when the grid fits one
-  // round of them, two otherwise (a 320-workgroup grid of 16-wave ones took
-  // two rounds: 38 us against 32 us with two phases, 10240x8192 at N = 8); N > 32 on large grids: 128-row workgroups with two
-  // bands per wave.  4 <= N <= 16 with at least 7/8 of a workgroup per CU:
-  // the same 64-row workgroups over one 16-column block (each X tile crosses
-  // L2 once per four bands: 8-24% faster than one band per workgroup at
-  // N = 8 / 16 on such grids, even at N = 4).  Otherwise N <= 16:
-  // workgroups of 8 K phases over one or two bands.
-  const int64_t wide_wgs = (int64_t)(M / 64) * split_k;
-  if (nb >= 2 || (N >= 4 && wide_wgs * 8 >= (int64_t)device_cu_count() * 7)) {
-    const bool ph4 = wide_wgs <= (int64_t)device_cu_count();
-    if (nb <= 1)
-      e = ph4 ? launch_rwide<1, 4, 4>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx)
-              : launch_rwide<1, 4, 2>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx);
-    else if (nb <= 2 && M % 128 == 0 && split_k <= 2 && (int64_t)(M / 128) * split_k >= 160)
-      // two bands per wave at 17 <= N <= 32 on large grids of one or two
-      // slices (28672 / 14336 rows: 3-5% faster; with four slices, and on
-      // 10240 rows, slower than one band per wave)
-      e = launch_rwide2<2, 8, 2>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k,
-                                 kb_per_split, fx);
-    else if (nb <= 2)
-      e = ph4 ? launch_rwide<2, 4, 4>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx)
-              : launch_rwide<2, 4, 2>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx);
-    else if (nb <= 4 && M % 128 == 0 && split_k <= 2 && (int64_t)(M / 128) * split_k >= 160)
-      // (with four slices one band per wave is faster: 8192 rows at N = 48 /
-      // 64, 83 -> 80 us)
-      e = launch_rwide2<4, 8, 2>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k,
-                                 kb_per_split, fx);
-    else if (nb <= 4)
-      e = ph4 ? launch_rwide<4, 4, 4>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx)
-              : launch_rwide<4, 4, 2>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx);
-    else if (M % 128 == 0 && (int64_t)(M / 128) * split_k * ((N + 127) / 128) >= 160)
-      // two bands per wave halve the LDS reads of X per record; they pay
-      // once the 128-row grid still has >= 160 workgroups (measured)
-      e = launch_rwide2<8, 8, 2>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k,
-                                 kb_per_split, fx);
-    else if (kb_per_split >= 32)
-      // three K phases (12 waves, 3 per SIMD, B fragments read next to
-      // their MFMAs) on slices of >= 32 tiles: 2-10% faster than two phases
-      // with the early B reads (4096-deep slices of 32 tiles: ~5%); on
-      // slices of 16 tiles the uneven phases cost about what they gain
-      e = launch_rwide<8, 4, 3>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx);
-    else
-      e = launch_rwide<8, 4, 2>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx);
-  } else {
-    // Two bands per wave halve the X bytes per record (the cost that grows
-    // with N) but also the grid: for N > 8 once the grid keeps at least
-    // 192 workgroups.  Workgroups of 4 waves (16 per CU, twice the K tiles
-    // per wave) instead of 8 for N > 1 on grids of >= 640 bands (measured:
-    // 1-5 us faster at N = 8 / 16 on 10240, 14336 and 28672 rows, slower on
-    // smaller grids) and for N = 1 on grids of >= 896 bands (14336 rows:
-    // 21.9 -> 19.6 us; 28672 rows: 0-2% faster; 10240 rows at N = 1 are
-    // 0.6 us slower with 4 waves).
-    const bool w4 = M / 16 >= (N > 1 ? 640 : 896);
-    if (N > 8 && M / 16 >= 384)
-      e = w4 ? launch_rgemm<2, 1, 4>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx)
-             : launch_rgemm<2, 1, 8>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx);
-    else
-      e = w4 ? launch_rgemm<1, 1, 4>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx)
-             : launch_rgemm<1, 1, 8>(st, d_fixed, d_exps, d_eoff, se, B, out, M, N, K, split_k, kb_per_split, fx);
-  }
+  hipError_t e = mm_kernel(M, N, K, split_k)
+                     .launch(st, d_fixed, d_exps, d_eoff, (int)start_exp, B, out, M, N, K, split_k,
+                             kb_per_split, fx);
   if (e != hipSuccess) return (int)e;
   if (split_k > 1 && !counters) {
     const int64_t mn = (int64_t)M * N;
