@@ -10,6 +10,7 @@ kernel_benchmark/bench_zipserv_decode_attention.py:337-354.  The compute is
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional
 
@@ -166,12 +167,8 @@ def _retiled_desc(c, *, name, device, batch_size, num_heads_k):
     bsr = c.rows // batch_size
     if bsr % num_heads_k:
         raise ValueError(f"{name}.rows must encode an integer rows-per-head for num_heads_k={num_heads_k}")
-    d = _lib.KVRetiled()
-    d.fixed, d.exps, d.eoff = _dptr(c.fixed), _dptr(c.exps), _dptr(c.eoff)
-    d.rows, d.cols = c.rows, c.cols
-    d.batch_stride_rows, d.head_stride_rows = bsr, bsr // num_heads_k
-    d.start_exp, d.layout = c.start_exp, LAYOUT_IDS[str(c.layout)]
-    return d
+    return _lib.KVRetiled(_dptr(c.fixed), _dptr(c.exps), _dptr(c.eoff), c.rows, c.cols, bsr,
+                          bsr // num_heads_k, c.start_exp, LAYOUT_IDS[str(c.layout)])
 
 
 def _normalize_zipserv_kv(desc, *, name: str, device, batch_size: int, num_heads_k: int):
@@ -280,7 +277,6 @@ def flash_attn_with_kvcache_zipserv(q, zipserv_k, zipserv_v, zipserv_num_heads_k
         wsb += int(L.zs_kv_retiled_staging_bytes(d.layout, d.rows, d.cols, zipserv_num_heads_k)
                    if retiled else L.zs_kv_staging_bytes(d.layout, d.rows, d.cols))
     ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device=q.device)
-    import ctypes
     fn_name = "zs_decode_attention_retiled" if retiled else "zs_decode_attention"
     check(fn_name, getattr(L, fn_name)(
         _stream(), _dptr(q3), ctypes.byref(dk), ctypes.byref(dv), _dptr(sl), int(seqlen_k), B, H,

@@ -148,18 +148,27 @@ def compress_host(a: np.ndarray, top=None, variant: str = "reuse_simd") -> HostC
 # --------------------------------------------------------------------------
 # Device codec (torch tensors on the GPU)
 # --------------------------------------------------------------------------
+_torch_module = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
 
 
 def _dptr(t) -> int:
-    return 0 if t is None else int(t.data_ptr())
+    return 0 if t is None else t.data_ptr()
 
 
 def _stream() -> int:
+    """The current device's current stream, without the Stream object that
+    torch.cuda.current_stream() builds (2.9 -> 0.3 us of a call; zipgemm 9.7
+    -> 6.9 us, compressed decode attention 17.1 -> 13.7 us on the host)."""
     torch = _torch()
-    return int(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 @dataclass
