@@ -92,10 +92,11 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const uint16_t* in, 
 // stride >= 32 and at most kSampleChunks chunks -- for the window guess of
 // the one-pass re-tiled encoder.  kSampleGroups workgroups each write their
 // own 256 bins (slice blockIdx.x of `slices`, no atomics, so nothing needs
-// zeroing first) and clear `zero` (the fused encoding pass's kVerifySlices
-// histogram slices, added to with atomics later) and *zero32 (when given:
-// the arrival counter of the offset scan).
-constexpr int kSampleStrideMin = 32, kSampleChunks = 128, kSampleGroups = 4;
+// zeroing first) and clear `zero` (the fused encoding pass's histogram slices,
+// added to with atomics later, and the sums of the offset scan) and *zero32
+// (when given: the scan's ticket).
+// (8 groups: 6.8 us for 512 KB; 4 took two rounds of loads and 9.0.)
+constexpr int kSampleStrideMin = 32, kSampleChunks = 128, kSampleGroups = 8;
 
 __host__ __device__ __forceinline__ int64_t sample_stride(int64_t nchunks) {
   const int64_t s = (nchunks + kSampleChunks - 1) / kSampleChunks;
@@ -106,11 +107,11 @@ __global__ __launch_bounds__(kHistThreads) void sample_hist_kernel(const uint16_
                                                                    int64_t nchunks,
                                                                    uint64_t zeros,
                                                                    uint64_t* slices,
-                                                                   uint64_t* zero,
+                                                                   uint64_t* zero, int nzero,
                                                                    int32_t* zero32) {
   __shared__ uint32_t h[kHistCopies * kHistPitch];
   for (int i = threadIdx.x; i < kHistCopies * kHistPitch; i += kHistThreads) h[i] = 0;
-  for (int i = blockIdx.x * kHistThreads + threadIdx.x; i < kVerifySlices * 256;
+  for (int i = blockIdx.x * kHistThreads + threadIdx.x; i < nzero;
        i += kSampleGroups * kHistThreads)
     zero[i] = 0;
   if (zero32 && blockIdx.x == 0 && threadIdx.x == 0) *zero32 = 0;
@@ -529,17 +530,18 @@ namespace zs {
 // Window guess from a sample of the input (chunks of 2048 elements, at most
 // kSampleChunks of them; a partial last chunk, when numel is not a multiple
 // of 2048, is not sampled; input 16-byte aligned) into `guess`; the per-workgroup
-// sample bins go to `sample` (kSampleGroups x 256), and `zero`
-// (kVerifySlices x 256 entries) and *zero32 (when given) are cleared on the way.
+// sample bins go to `sample` (kSampleGroups x 256), and `zero` (nzero entries)
+// and *zero32 (when given) are cleared on the way.
 // `zeros`: elements of the encoded matrix that are not in `in` (zero padding),
 // counted in the sample in proportion.
 hipError_t launch_window_sample(hipStream_t st, const uint16_t* in, int64_t numel, int64_t zeros,
-                                bool weights_rule, uint64_t* sample, uint64_t* zero,
+                                bool weights_rule, uint64_t* sample, uint64_t* zero, int nzero,
                                 int32_t* guess, int32_t* zero32) {
   const int64_t nchunks = numel / 2048, stride = sample_stride(nchunks);
   const int64_t sampled = (nchunks + stride - 1) / stride * 2048;
   hipLaunchKernelGGL(sample_hist_kernel, dim3(kSampleGroups), dim3(kHistThreads), 0, st, in,
-                     nchunks, (uint64_t)((double)zeros * sampled / numel), sample, zero, zero32);
+                     nchunks, (uint64_t)((double)zeros * sampled / numel), sample, zero, nzero,
+                     zero32);
   if (weights_rule)
     hipLaunchKernelGGL((select_weights_kernel<uint64_t, kSampleGroups>), dim3(1), dim3(256), 0, st,
                        sample, nullptr, guess, nullptr, nullptr);

@@ -178,15 +178,9 @@ __device__ __forceinline__ int block256_exclusive(int v, int& total) {
   return before + incl - v;
 }
 
-// Sum of each kScanTile-record tile into eoff[tile * kScanTile].  With
-// `arrive` (a counter that is zero on entry), the workgroup that arrives last
-// also turns the tile sums into exclusive tile offsets and writes the total
-// (the work of rscan_tiles_kernel, one launch fewer), then returns the
-// counter to zero; the sums travel between workgroups through device-scope
-// stores and loads, as in splitk_finish.
+// Sum of each kScanTile-record tile into eoff[tile * kScanTile].
 __global__ __launch_bounds__(256) void rscan_reduce_kernel(const int32_t* counts, int64_t n,
-                                                           int32_t* eoff, int32_t* arrive,
-                                                           int64_t* total_out) {
+                                                           int32_t* eoff) {
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
   int s = 0;
 #pragma unroll
@@ -196,36 +190,7 @@ __global__ __launch_bounds__(256) void rscan_reduce_kernel(const int32_t* counts
   }
   int total;
   block256_exclusive(s, total);
-  if (!arrive) {
-    if (threadIdx.x == 0) eoff[base] = total;
-    return;
-  }
-  __shared__ int last;
-  if (threadIdx.x == 0) {
-    __hip_atomic_store(&eoff[base], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __builtin_amdgcn_s_waitcnt(0);  // the store is performed before the arrival counts
-    last = __hip_atomic_fetch_add(arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-           (int)gridDim.x - 1;
-  }
-  __syncthreads();
-  if (!last) return;
-  const int64_t ntiles = gridDim.x;
-  int64_t carry = 0;
-  for (int64_t t0 = 0; t0 < ntiles; t0 += 256) {
-    const int64_t tile = t0 + threadIdx.x;
-    const int v = tile < ntiles ? __hip_atomic_load(&eoff[tile * kScanTile], __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT)
-                                : 0;
-    int chunk;
-    const int ex = block256_exclusive(v, chunk);
-    if (tile < ntiles) eoff[tile * kScanTile] = (int32_t)(carry + ex);
-    carry += chunk;
-  }
-  if (threadIdx.x == 0) {
-    eoff[n] = (int32_t)carry;
-    *total_out = carry;
-    __hip_atomic_store(arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (threadIdx.x == 0) eoff[base] = total;
 }
 
 __global__ __launch_bounds__(1024) void rscan_tiles_kernel(int32_t* eoff, int64_t n,
@@ -279,16 +244,77 @@ __global__ __launch_bounds__(256) void rscan_write_kernel(const int32_t* counts,
   }
 }
 
+// The whole scan in one launch, for at most kScanFlags tiles.  A workgroup takes
+// the next tile by a ticket (`ticket`, zero on entry and again on exit),
+// publishes the tile's sum + 1 in sums[tile] (zeroed by the caller), adds up the
+// sums of the tiles before it, waiting for those not yet published, and writes
+// its offsets.  Every wait ends: the tiles waited for have smaller tickets, so
+// their workgroups run already, and they publish before they wait.  The sums
+// travel between workgroups through device-scope stores and loads, as in
+// splitk_finish.  57344 records: 5.2 us, a launch for the sums and one for the
+// offsets 4.5 + 4.4 and the gap between them.
+constexpr int kScanFlags = 4096;
+
+__global__ __launch_bounds__(256) void rscan_kernel(const int32_t* counts, int64_t n,
+                                                    int32_t* eoff, int64_t* total_out,
+                                                    int32_t* sums, int32_t* ticket) {
+  __shared__ int tile_s;
+  __shared__ int64_t ws[4];
+  if (threadIdx.x == 0) {
+    tile_s = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tile_s == (int)gridDim.x - 1)  // the last ticket
+      __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  const int tile = tile_s;
+  const int64_t i0 = (int64_t)tile * kScanTile + 4 * threadIdx.x;
+  int c[4], s = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    c[j] = i0 + j < n ? counts[i0 + j] : 0;
+    s += c[j];
+  }
+  int total;
+  const int ex = block256_exclusive(s, total);
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&sums[tile], total + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int64_t before = 0;
+  for (int t = threadIdx.x; t < tile; t += 256) {
+    int v;
+    while ((v = __hip_atomic_load(&sums[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
+      __builtin_amdgcn_s_sleep(1);
+    before += v - 1;
+  }
+#pragma unroll
+  for (int d = 32; d; d >>= 1) before += __shfl_xor(before, d);
+  if (lane_id() == 0) ws[threadIdx.x >> 6] = before;
+  __syncthreads();
+  const int64_t off = ws[0] + ws[1] + ws[2] + ws[3];
+  int run = (int)off + ex;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (i0 + j < n) eoff[i0 + j] = run;
+    run += c[j];
+  }
+  if (tile == (int)gridDim.x - 1 && threadIdx.x == 0) {
+    eoff[n] = (int32_t)(off + total);
+    *total_out = off + total;
+  }
+}
+
 // Exclusive scan of the per-record outlier counts into eoff (n + 1 entries,
-// eoff[n] = *total).  `arrive`: a zeroed counter that lets the reduce kernel
-// scan the tile sums itself (two launches instead of three).
+// eoff[n] = *total), in one launch with `sums` (kScanFlags zeroed entries) and a
+// zeroed `ticket`, unless there are more tiles than that.
 static void launch_rscan(hipStream_t st, const int32_t* counts, int64_t n, int32_t* eoff,
-                         int64_t* total, int32_t* arrive = nullptr) {
+                         int64_t* total, int32_t* sums = nullptr, int32_t* ticket = nullptr) {
   const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL(rscan_reduce_kernel, dim3((unsigned)tiles), dim3(256), 0, st, counts, n, eoff,
-                     arrive, total);
-  if (!arrive)
-    hipLaunchKernelGGL(rscan_tiles_kernel, dim3(1), dim3(1024), 0, st, eoff, n, total);
+  if (sums && tiles <= kScanFlags) {
+    hipLaunchKernelGGL(rscan_kernel, dim3((unsigned)tiles), dim3(256), 0, st, counts, n, eoff, total,
+                       sums, ticket);
+    return;
+  }
+  hipLaunchKernelGGL(rscan_reduce_kernel, dim3((unsigned)tiles), dim3(256), 0, st, counts, n, eoff);
+  hipLaunchKernelGGL(rscan_tiles_kernel, dim3(1), dim3(1024), 0, st, eoff, n, total);
   hipLaunchKernelGGL(rscan_write_kernel, dim3((unsigned)tiles), dim3(256), 0, st, counts, n, eoff);
 }
 
@@ -791,7 +817,7 @@ int device_cu_count();  // zs_gemm.hip
 // window of a full histogram with a flag saying whether it differs.
 hipError_t launch_window_sample(hipStream_t st, const uint16_t* in, int64_t numel,
                                 int64_t zeros, bool weights_rule, uint64_t* sample, uint64_t* zero,
-                                int32_t* guess, int32_t* zero32);
+                                int nzero, int32_t* guess, int32_t* zero32);
 
 
 __global__ __launch_bounds__(kDecWaves * 64) void rdecompress_kernel(const uint8_t* fixed,
@@ -2337,12 +2363,14 @@ extern "C" int zs_compress_retiled_fixed_gpu(void* stream, const uint16_t* d_inp
   return status_of(hipGetLastError());
 }
 
-// d_work: kHistSlices histogram slices of the encoding pass, as many of the
-// sample, the guessed window and the flag that says whether the full
-// histogram's window differs.
-constexpr int kWorkSample = kHistSlices * 256 * 8, kWorkGuess = 2 * kWorkSample,
-              kWorkDiffers = kWorkGuess + 32, kWorkArrive = kWorkDiffers + 4;
-static_assert(kWorkArrive + 4 <= ZS_RETILED_AUTO_WORK_BYTES, "auto encoder scratch");
+// d_work: kHistSlices histogram slices of the encoding pass, the sums of the
+// offset scan's tiles, the histograms of the sample, the guessed window, the flag
+// that says whether the full histogram's window differs, and the scan's ticket.
+constexpr int kWorkSums = kHistSlices * 256 * 8, kWorkSample = kWorkSums + 4 * kScanFlags,
+              kWorkGuess = 2 * kWorkSums, kWorkDiffers = kWorkGuess + 32,
+              kWorkTicket = kWorkDiffers + 4;
+static_assert(kWorkSample + 8 * 256 * 8 <= kWorkGuess, "sample histograms");  // kSampleGroups
+static_assert(kWorkTicket + 4 <= ZS_RETILED_AUTO_WORK_BYTES, "auto encoder scratch");
 
 __global__ void zero_i32_kernel(int32_t* p, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2371,16 +2399,17 @@ static int retiled_auto(void* stream, const Src& src, const uint16_t* dense, int
   uint64_t* sample = reinterpret_cast<uint64_t*>(d_work + kWorkSample);
   int32_t* guess = reinterpret_cast<int32_t*>(d_work + kWorkGuess);
   int32_t* differs = reinterpret_cast<int32_t*>(d_work + kWorkDiffers);
-  int32_t* arrive = reinterpret_cast<int32_t*>(d_work + kWorkArrive);  // the scan's counter
+  int32_t* sums = reinterpret_cast<int32_t*>(d_work + kWorkSums);
+  int32_t* ticket = reinterpret_cast<int32_t*>(d_work + kWorkTicket);
   if (d_guess) {
     // the caller's window as the guess: only the histogram slices and the
-    // scan's counter need clearing (one fill over the start of d_work)
-    hipLaunchKernelGGL(zero_i32_kernel, dim3((kWorkArrive / 4 + 1 + 255) / 256), dim3(256), 0, st,
-                       reinterpret_cast<int32_t*>(d_work), (int64_t)(kWorkArrive / 4 + 1));
+    // scan's sums and ticket need clearing (one fill of d_work)
+    hipLaunchKernelGGL(zero_i32_kernel, dim3((kWorkTicket / 4 + 1 + 255) / 256), dim3(256), 0, st,
+                       reinterpret_cast<int32_t*>(d_work), (int64_t)(kWorkTicket / 4 + 1));
     guess = const_cast<int32_t*>(d_guess);
   } else {
     const hipError_t e = launch_window_sample(st, dense, n, zeros, weights, sample, slices,
-                                              guess, arrive);
+                                              kWorkSample / 8, guess, ticket);
     if (e != hipSuccess) return status_of(e);
   }
   const int hist_grid = r_grid(nrec, 4);
@@ -2392,7 +2421,7 @@ static int retiled_auto(void* stream, const Src& src, const uint16_t* dense, int
                      dim3(std::min(r_grid(nrec, 4), device_cu_count() * 2)), dim3(256), 0, st, src,
                      M, K, d_top, d_fixed, d_counts, d_tmp, nullptr,
                      nullptr, WindowCheck{slices, d_hist, d_top, guess, differs, weights ? 1 : 0});
-  launch_rscan(st, d_counts, nrec, d_eoff, d_total, arrive);
+  launch_rscan(st, d_counts, nrec, d_eoff, d_total, sums, ticket);
   return status_of(hipGetLastError());
 }
 
