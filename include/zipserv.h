@@ -373,8 +373,13 @@ typedef struct zs_kv_compressed {
  * q, out: [batch][num_heads][head_dim] bf16, 16-byte aligned.  L_b = cache_seqlens[b] (device
  * int32 [batch]) or seqlen_k when cache_seqlens is NULL.  softmax_lse
  * (optional, [batch][num_heads] fp32) is the natural-log normaliser.
- * num_splits = 0 picks a split of the sequence across workgroups; splits > 1
- * need `workspace` of zs_decode_attention_workspace_bytes bytes.
+ * num_splits = 0 picks the splits of the sequences across workgroups; splits > 1
+ * need `workspace` of zs_decode_attention_workspace_bytes bytes.  The picked
+ * splits depend on the batch and on seqlen_k, and over compressed caches with
+ * cache_seqlens also on all the lengths, so the rounding of one sequence's
+ * result may change with its neighbours' lengths; num_splits > 0 cuts every
+ * sequence alike.  cache_seqlens is read by the attention kernel alone (what is
+ * queued on it behind the call does not change the result).
  * Layouts (flash.h:19-20): HEAD_MAJOR caches (row (b*Hkv + h)*head_stride +
  * t) are decoded inside the attention kernel; TOKEN_MAJOR caches (row
  * b*batch_stride + t*Hkv + h) run staged -- both are first decompressed into

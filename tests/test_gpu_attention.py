@@ -26,7 +26,8 @@ def _bf16_f32(a):
 
 
 def _run(torch_cuda, B, T, Hkv, H, seqlens=None, splits=0, seed=0, q_zero=False, retiled=False,
-         layout="by_kv_head"):
+         layout="by_kv_head", passed=None):
+    """passed: the lengths that the kernels are given, where they are not seqlens."""
     import zipserv_asplos26_amd.attention as za
     torch = torch_cuda
     rng = np.random.default_rng(seed)
@@ -39,7 +40,8 @@ def _run(torch_cuda, B, T, Hkv, H, seqlens=None, splits=0, seed=0, q_zero=False,
     kd, vd, qd = to_torch_bf16(k), to_torch_bf16(v), to_torch_bf16(q)
     ck = za.compress_kv(kd, layout=layout, retiled=retiled)
     cv = za.compress_kv(vd, layout=layout, retiled=retiled)
-    sl = None if seqlens is None else torch.tensor(seqlens, dtype=torch.int32, device="cuda")
+    passed = seqlens if passed is None else passed
+    sl = None if passed is None else torch.tensor(passed, dtype=torch.int32, device="cuda")
     out, lse = za.flash_attn_with_kvcache_zipserv(
         qd.view(B, 1, H, D), ck, cv, Hkv, T, cache_seqlens=sl, num_splits=splits,
         return_softmax_lse=True)

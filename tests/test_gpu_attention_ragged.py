@@ -1,8 +1,8 @@
-"""Decode attention over ragged batches with automatic splits: the splits
-follow the sequences' lengths (one chunk for the whole call, as many splits as
-a sequence needs), in every mode, against the fp64 oracle within
-zs_testutil.attention_tolerance, and compressed against dense bit for bit where
-both cut the same pieces."""
+"""Decode attention over ragged batches with automatic splits, against the fp64
+oracle within zs_testutil.attention_tolerance: equal splits (short sequences),
+compressed against dense bit for bit where both cut the same pieces, and splits
+that follow the sequences' lengths (one chunk for the whole call, as many splits
+as a sequence needs), which long splits of a compressed cache have."""
 import numpy as np
 import pytest
 
@@ -34,7 +34,7 @@ CASES = [
 @pytest.mark.parametrize("retiled", [False, True])
 def test_ragged_head_major(torch_cuda, B, T, lens, retiled):
     used = [min(v, T) for v in lens]
-    res = _run(torch_cuda, B, T, 2, 8, seqlens=used, splits=0, seed=B, retiled=retiled)
+    res = _run(torch_cuda, B, T, 2, 8, seqlens=used, splits=0, seed=B, retiled=retiled, passed=lens)
     # the dense kernel cuts the same pieces where its split count is the same
     # (short sequences: the minimum split length decides in both)
     _check(res, used, exact=B <= 5 and T < 1000)
@@ -44,12 +44,42 @@ def test_ragged_head_major(torch_cuda, B, T, lens, retiled):
 def test_ragged_token_major(torch_cuda, B, T, lens):
     used = [min(v, T) for v in lens]
     _check(_run(torch_cuda, B, T, 8, 16, seqlens=used, splits=0, seed=B + 1, retiled=True,
-                layout="token_major"), used, exact=False)
+                layout="token_major", passed=lens), used, exact=False)
+
+
+# (layout, B, T, Hkv, H, lengths), all with splits that follow the lengths
+BALANCED = [
+    ("by_kv_head", 2, 9000, 8, 64, [9000, 1]),                # nearly all pieces in one sequence
+    ("by_kv_head", 3, 9000, 4, 8, [0, 9000, 20000]),          # an empty one, one past the cache
+    ("by_kv_head", 4, 16000, 2, 8, [0, 0, -7, 0]),            # no tokens at all
+    ("by_kv_head", 64, 2000, 2, 8, _lens(64, 2000, 1)),       # one wave's lanes of lengths
+    ("by_kv_head", 65, 1700, 2, 8, _lens(65, 1700, 2)),       # one more
+    ("by_kv_head", 256, 1000, 1, 4, _lens(256, 1000, 3)),     # as many as the plan takes
+    ("by_kv_head", 154, 960, 5, 10, _lens(154, 960, 4)),      # one wave an item: idle and busy waves
+                                                              # share the last workgroups
+    ("token_major", 3, 9000, 8, 16, [9000, 16, 17]),
+    ("token_major", 2, 700, 8, 16, [700, 90]),                # one workgroup a CU
+    ("token_major", 64, 512, 8, 8, _lens(64, 512, 5)),
+    ("token_major", 65, 530, 8, 8, _lens(65, 530, 6)),
+    ("token_major", 200, 500, 8, 8, _lens(200, 500, 7)),      # fewer pieces than batch * splits
+    ("token_major", 256, 520, 8, 8, _lens(256, 520, 8)),
+]
+
+
+@pytest.mark.parametrize("layout,B,T,Hkv,H,lens", BALANCED)
+def test_splits_that_follow_the_lengths(torch_cuda, layout, B, T, Hkv, H, lens):
+    used = [min(max(v, 0), T) for v in lens]
+    _check(_run(torch_cuda, B, T, Hkv, H, seqlens=used, splits=0, seed=B, retiled=True,
+                layout=layout, passed=lens), used, exact=False)
+
+
+@pytest.mark.parametrize("B,T,lens", [(3, 9000, [9000, 40, 5000]), (40, 1600, _lens(40, 1600, 9))])
+def test_splits_that_follow_the_lengths_canonical(torch_cuda, B, T, lens):
+    _check(_run(torch_cuda, B, T, 2, 8, seqlens=lens, splits=0, seed=B), lens, exact=False)
 
 
 def test_ragged_large_grid(torch_cuda):
-    # one wave per item in the head-major kernel (>= 2048 items), the last
-    # workgroups past the last piece
+    # a full round of shared items, the last workgroups past the last piece
     lens = [4096, 100, 2048, 3000, 1, 0, 4000, 511] * 2
     _check(_run(torch_cuda, 16, 4096, 8, 32, seqlens=lens, splits=0, seed=9, retiled=True), lens,
            exact=False)

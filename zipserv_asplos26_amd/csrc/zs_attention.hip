@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "../../include/zipserv.h"
 #include "zs_device.hpp"
@@ -82,16 +83,19 @@ struct AttnParams {
   float* lse;                   // [B][H] or null
   float* ws_o;                  // [B][H][splits][D]   (splits > 1)
   float* ws_ml;                 // [B][H][splits][2]
+  int2* plan;                   // [B] (first piece, pieces) of each sequence (balanced)
   const int32_t* seqlens;       // [B] or null
   int seqlen_k, batch, heads, heads_k, group, splits, chunk;
   int balanced;                 // splits follow the sequences' lengths (AttnSeq)
+  FastDiv pieces, spare;        // balanced: at most pieces.d of them, > batch and <= batch *
+                                // splits; spare.d: pieces.d - batch
   int shared;                   // a workgroup's waves share one item
   float scale_log2;             // softmax_scale * log2(e)
 };
 
 // The place of one split among a call's sequences: split `sp` of sequence
 // `b`, which has `n` splits of `chunk` tokens, the first of them the call's
-// `first`-th.
+// `first`-th (n and first: balanced splits only).
 struct AttnSeq {
   int b, sp, n, first, chunk, len;
 };
@@ -102,89 +106,90 @@ __device__ __forceinline__ int attn_len(const AttnParams& p, int b) {
 }
 
 // Balanced splits (p.balanced): equal splits of every sequence make the
-// longest one decide a ragged batch's time -- 32 sequences of 125..4000
-// tokens, 16 splits each, left half of the workgroups with half the tokens or
-// fewer (token-major, 64 / 8 heads, 201 MB: 78.3 us, 56.9 us with the splits
-// below; equal lengths run as before).  Here the chunk is one for the whole call, the
-// smallest number of 16-token steps that cuts the sequences into at most
-// batch * splits pieces, and a sequence has as many splits as it needs.  With
-// equal lengths that is the even split.  Every wave finds its own piece from
-// the lengths: C >= ceil(S / G) for S steps and G pieces, and ceil(S / (G -
-// batch)) always fits, so the search between the two takes a step or two.
-__device__ __forceinline__ int attn_pieces(const AttnParams& p, int c) {
-  int sum = 0;
-  for (int b0 = 0; b0 < p.batch; b0 += 64) {
-    const int b = b0 + lane_id();
-    const int steps = b < p.batch ? (attn_len(p, b) + 15) >> 4 : 0;
-    sum += (steps + c - 1) / c;
-  }
-  return __builtin_amdgcn_readlane(wave_inclusive_scan(sum), 63);
+// longest one decide a ragged batch's time.  Here the chunk is one for the whole
+// call, a number of 16-token steps that cuts the sequences into at most
+// p.pieces pieces, and a sequence has as many splits as it needs; with equal
+// lengths that is the even split.  Every wave of the attention kernel finds its
+// own piece from the lengths, and the first one writes every sequence's pieces
+// to p.plan for the merge, which so reads the cut that the kernel made, whatever
+// is queued on the lengths between the two launches.  The lengths are loaded
+// once, into registers (kPlanChunks x 64 of them), and the search takes at most
+// kPlanTries sums over them: a merge that found the plan by itself, and loads of
+// the lengths in every step of the search, cost 3 us of a call of 16 sequences
+// and half the time of one of 192.  Token-major cache, 32 sequences of 125..4000
+// tokens, 64 / 8 heads: 81.4 us with equal splits, 56.6 with these (201 MB).
+constexpr int kPlanChunks = 4, kPlanTries = 4;
+constexpr int kPlanSeqs = kPlanChunks * 64;
+
+__device__ __forceinline__ int wave_total(int v) {
+  return __builtin_amdgcn_readlane(wave_inclusive_scan(v), 63);
 }
 
-__device__ __forceinline__ int attn_balanced_steps(const AttnParams& p) {
-  const int G = p.batch * p.splits;
-  const int S = attn_pieces(p, 1);
-  int lo = max((S + G - 1) / G, 1);
-  int hi = max((S + G - p.batch - 1) / (G - p.batch), lo);  // splits > 1: G > batch
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (attn_pieces(p, mid) <= G)
-      hi = mid;
-    else
-      lo = mid + 1;
+// Piece u (wave-uniform) of the balanced cut, b = -1 past the last one; u == 0
+// with `write` also writes p.plan.
+__device__ __forceinline__ AttnSeq attn_seq_of_piece(const AttnParams& p, int u, bool write) {
+  int len[kPlanChunks];
+#pragma unroll
+  for (int i = 0; i < kPlanChunks; ++i) {
+    const int b = 64 * i + lane_id();
+    len[i] = 64 * i < p.batch && b < p.batch ? attn_len(p, b) : 0;
   }
-  return lo;
-}
-
-// Piece u (wave-uniform) of the balanced cut, b = -1 past the last one.
-__device__ __forceinline__ AttnSeq attn_seq_of_piece(const AttnParams& p, int u) {
-  const int c = attn_balanced_steps(p);
-  AttnSeq s{-1, 0, 0, 0, 16 * c, 0};
+  FastDiv chunk{1, 0};  // steps a piece
+  auto pieces = [&](int i) {  // of the i-th 64 sequences' own one
+    return (int)chunk.div((uint32_t)((len[i] + 15) >> 4) + chunk.d - 1);
+  };
+  auto total = [&]() {
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < kPlanChunks; ++i)
+      if (64 * i < p.batch) s += pieces(i);
+    return (uint32_t)wave_total(s);
+  };
+  // ceil(S / G) for S steps and G pieces is the least that can do, and ceil(S /
+  // (G - batch)) always does; in between, a cut into P > G pieces asks for about
+  // P / G times its chunk.
+  const uint32_t S = total(), G = p.pieces.d;
+  const uint32_t most = max(p.spare.div(S + p.spare.d - 1), 1u);
+  uint32_t c = max(p.pieces.div(S + G - 1), 1u);
+  for (int i = 0;; ++i) {
+    chunk = FastDiv::of(c);
+    if (c >= most) break;
+    const uint32_t P = total();
+    if (P <= G) break;
+    c = i + 1 < kPlanTries ? min(most, max(c + 1, (uint32_t)((float)c * (float)P / (float)G))) : most;
+  }
+  AttnSeq s{-1, 0, 0, 0, 16 * (int)c, 0};
   int base = 0;
-  for (int b0 = 0; b0 < p.batch; b0 += 64) {
-    const int b = b0 + lane_id();
-    const int len = b < p.batch ? attn_len(p, b) : 0;
-    const int n = (((len + 15) >> 4) + c - 1) / c;
-    const int incl = wave_inclusive_scan(n);
-    const uint64_t hit = __builtin_amdgcn_ballot_w64(u >= base + incl - n && u < base + incl);
-    if (hit) {
-      const int j = __builtin_ctzll(hit);
-      s.b = b0 + j;
-      s.n = __builtin_amdgcn_readlane(n, j);
-      s.first = base + __builtin_amdgcn_readlane(incl, j) - s.n;
-      s.sp = u - s.first;
-      s.len = __builtin_amdgcn_readlane(len, j);
-      break;
+  bool found = false;
+  // (unrolled: the lengths are in registers)
+#pragma unroll
+  for (int i = 0; i < kPlanChunks; ++i) {
+    if (64 * i < p.batch && (write || !found)) {
+      const int n = pieces(i);
+      const int incl = wave_inclusive_scan(n);
+      const int first = base + incl - n;
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(u >= first && u < first + n);
+      if (hit) {
+        const int j = __builtin_ctzll(hit);
+        found = true;
+        s.b = 64 * i + j;
+        s.n = __builtin_amdgcn_readlane(n, j);
+        s.first = __builtin_amdgcn_readlane(first, j);
+        s.sp = u - s.first;
+        s.len = __builtin_amdgcn_readlane(len[i], j);
+      }
+      if (write && 64 * i + lane_id() < p.batch) p.plan[64 * i + lane_id()] = make_int2(first, n);
+      base += __builtin_amdgcn_readlane(incl, 63);
     }
-    base += __builtin_amdgcn_readlane(incl, 63);
-  }
-  return s;
-}
-
-// The pieces of sequence b (their number and the first one).
-__device__ __forceinline__ AttnSeq attn_seq_of_batch(const AttnParams& p, int bq) {
-  const int c = attn_balanced_steps(p);
-  AttnSeq s{bq, 0, 0, 0, 16 * c, 0};
-  int base = 0;
-  for (int b0 = 0; b0 < p.batch; b0 += 64) {
-    const int b = b0 + lane_id();
-    const int len = b < p.batch ? attn_len(p, b) : 0;
-    const int n = (((len + 15) >> 4) + c - 1) / c;
-    const int incl = wave_inclusive_scan(n);
-    if (bq < b0 + 64) {
-      s.n = __builtin_amdgcn_readlane(n, bq - b0);
-      s.first = base + __builtin_amdgcn_readlane(incl, bq - b0) - s.n;
-      break;
-    }
-    base += __builtin_amdgcn_readlane(incl, 63);
   }
   return s;
 }
 
 // Partial-result slot of split sp of (b, head): the splits of one (b, head)
-// one after another, or with balanced splits the heads of one piece.
+// one after another.
+template <bool kBalanced>
 __device__ __forceinline__ int64_t attn_slot(const AttnParams& p, const AttnSeq& s, int head) {
-  return p.balanced ? (int64_t)(s.first + s.sp) * p.heads + head
+  return kBalanced ? (int64_t)s.first * p.heads + head * s.n + s.sp
                     : ((int64_t)s.b * p.heads + head) * p.splits + s.sp;
 }
 
@@ -329,7 +334,9 @@ __device__ __forceinline__ int kv_median(int rowbase, int med) {
 // The re-tiled mode asks for three waves per SIMD: the compiler then keeps
 // the MFMA accumulators in ordinary VGPRs (140 in all, no spills) instead of
 // splitting 135 VGPRs + 36 AGPRs, which allowed only two.
-template <int kMode, int kWpi>
+// kBalanced: splits follow the lengths (instances of their own: with the plan's
+// code in every start-up, calls without a plan took 0.3-0.6 us longer).
+template <int kMode, int kWpi, bool kBalanced>
 __global__ __launch_bounds__((kWpi == 1 ? kAttnWaves : kWpi) * 64,
                              kMode == kModeRetiled ? 3 : 1) void attn_kernel(AttnParams p) {
   constexpr bool kDense = kMode == kModeDense || kMode == kModePaged;
@@ -361,9 +368,9 @@ __global__ __launch_bounds__((kWpi == 1 ? kAttnWaves : kWpi) * 64,
   AttnSeq sq;
   int h;
   bool idle = item0 >= nitems;
-  if (p.balanced) {
+  if constexpr (kBalanced) {
     // the splits of one head of one sequence one after another
-    sq = attn_seq_of_piece(p, item / p.heads_k);
+    sq = attn_seq_of_piece(p, item / p.heads_k, item0 == 0 && (kWpi == 1 || w == 0));
     if (sq.b < 0) {  // past the last piece: no tokens, nothing written
       if constexpr (kMode != kModeRetiled) return;  // uniform when kWpi > 1
       idle = true;
@@ -689,7 +696,7 @@ __global__ __launch_bounds__((kWpi == 1 ? kAttnWaves : kWpi) * 64,
             A.l_run > 0.f ? (A.m_run + __log2f(A.l_run)) * 0.6931471805599453f : -INFINITY;
     }
   } else if (own) {
-    const int64_t slot = attn_slot(p, sq, head);
+    const int64_t slot = attn_slot<kBalanced>(p, sq, head);
     float* wo = p.ws_o + slot * kHeadDim + d0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(wo + 16 * i) = A.O[i];
@@ -745,7 +752,7 @@ constexpr int tm_lds() {
   return (int)sizeof(RTables) + kTmWaves * 2 * kExpStage + (D == 8 ? 4 : 2) * kTmPhase;
 }
 
-template <int D>
+template <int D, bool kBalanced>
 __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(AttnParams p) {
   static_assert(D % 4 == 0, "the ring holds whole steps");
   constexpr bool kPair = D == 8;
@@ -756,8 +763,8 @@ __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(
   const int l = lane_id();
   const int item = blockIdx.x;
   AttnSeq sq;
-  if (p.balanced) {
-    sq = attn_seq_of_piece(p, item);
+  if constexpr (kBalanced) {
+    sq = attn_seq_of_piece(p, item, item == 0 && w == 0);
     if (sq.b < 0) return;  // uniform: past the last piece
   } else {
     sq.chunk = p.chunk;
@@ -971,7 +978,7 @@ __global__ __launch_bounds__(kTmWaves * 64, D == 4 ? 4 : 2) void attn_tm_kernel(
             A.l_run > 0.f ? (A.m_run + __log2f(A.l_run)) * 0.6931471805599453f : -INFINITY;
     }
   } else if (own) {
-    const int64_t slot = attn_slot(p, sq, head);
+    const int64_t slot = attn_slot<kBalanced>(p, sq, head);
     float* wo = p.ws_o + slot * kHeadDim + d0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(wo + 16 * i) = A.O[i];
@@ -1008,38 +1015,36 @@ __device__ __forceinline__ float block_reduce(float x, bool is_max, float* red) 
   return r;
 }
 
-template <int W>
+template <int W, bool kBalanced>
 __global__ __launch_bounds__(W * 64) void attn_combine_kernel(AttnParams p) {
   constexpr int NT = W * 64;
   __shared__ float sc[kCombineChunk];
   __shared__ float red[W];
   __shared__ float2 part[W - 1][64];
   const int bh = blockIdx.x;
-  const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  // the partials of this (batch, head): S of them, `step` slots apart
-  int S = p.splits, step = 1;
+  // (w uniform: the partials' addresses are scalar; 80 -> 46 VGPRs with the plan)
+  const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
+  // the partials of this (batch, head): S of them
+  int S = p.splits;
   int64_t slot0 = (int64_t)bh * S;
-  if (p.balanced) {
+  if constexpr (kBalanced) {
     const int b = bh / p.heads;
-    const AttnSeq sq = attn_seq_of_batch(p, b);
-    S = sq.n;
-    step = p.heads;
-    slot0 = (int64_t)sq.first * p.heads + (bh - b * p.heads);
+    const int2 own = p.plan[b];
+    S = __builtin_amdgcn_readfirstlane(own.y);
+    slot0 = (int64_t)__builtin_amdgcn_readfirstlane(own.x) * p.heads + (int64_t)(bh - b * p.heads) * S;
   }
   const float* ml = p.ws_ml + slot0 * 2;
   const float* wo = p.ws_o + slot0 * kHeadDim + 2 * l;
-  const int64_t ostep = (int64_t)step * kHeadDim;
-  const int mstep = 2 * step;
   float2 x[8];
   {
     const int n = min(S, kCombineChunk);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      x[j] = 8 * w + j < n ? *reinterpret_cast<const float2*>(wo + (int64_t)(8 * w + j) * ostep)
+      x[j] = 8 * w + j < n ? *reinterpret_cast<const float2*>(wo + (int64_t)(8 * w + j) * kHeadDim)
                            : float2{0.f, 0.f};
   }
   float m = -INFINITY;
-  for (int s = t; s < S; s += NT) m = fmaxf(m, ml[(int64_t)mstep * s]);
+  for (int s = t; s < S; s += NT) m = fmaxf(m, ml[2 * s]);
   m = block_reduce<W>(m, true, red);
   const float m_use = m == -INFINITY ? 0.f : m;
   float lpart = 0.f;
@@ -1047,18 +1052,18 @@ __global__ __launch_bounds__(W * 64) void attn_combine_kernel(AttnParams p) {
   for (int c0 = 0; c0 < S; c0 += kCombineChunk) {
     const int n = min(S - c0, kCombineChunk);
     for (int i = t; i < n; i += NT) {
-      const float2 e = *reinterpret_cast<const float2*>(ml + (int64_t)mstep * (c0 + i));
+      const float2 e = *reinterpret_cast<const float2*>(ml + 2 * (c0 + i));
       const float wgt = e.y > 0.f ? __builtin_amdgcn_exp2f(e.x - m_use) : 0.f;
       sc[i] = wgt;
       lpart += e.y * wgt;
     }
     __syncthreads();
-    const float* wc = wo + (int64_t)c0 * ostep;
+    const float* wc = wo + (int64_t)c0 * kHeadDim;
     for (int i0 = 8 * w; i0 < n; i0 += 8 * W) {
       if (c0 > 0 || i0 > 8 * w) {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          x[j] = i0 + j < n ? *reinterpret_cast<const float2*>(wc + (int64_t)(i0 + j) * ostep)
+          x[j] = i0 + j < n ? *reinterpret_cast<const float2*>(wc + (int64_t)(i0 + j) * kHeadDim)
                             : float2{0.f, 0.f};
       }
 #pragma unroll
@@ -1088,10 +1093,18 @@ __global__ __launch_bounds__(W * 64) void attn_combine_kernel(AttnParams p) {
 }
 
 static hipError_t launch_combine(hipStream_t st, const AttnParams& p) {
-  if (p.splits > 32)
-    hipLaunchKernelGGL(attn_combine_kernel<16>, dim3(p.batch * p.heads), dim3(16 * 64), 0, st, p);
-  else
-    hipLaunchKernelGGL(attn_combine_kernel<4>, dim3(p.batch * p.heads), dim3(4 * 64), 0, st, p);
+  const dim3 grid(p.batch * p.heads);
+  if (p.balanced) {
+    if (p.splits > 32)
+      hipLaunchKernelGGL((attn_combine_kernel<16, true>), grid, dim3(16 * 64), 0, st, p);
+    else
+      hipLaunchKernelGGL((attn_combine_kernel<4, true>), grid, dim3(4 * 64), 0, st, p);
+  } else {
+    if (p.splits > 32)
+      hipLaunchKernelGGL((attn_combine_kernel<16, false>), grid, dim3(16 * 64), 0, st, p);
+    else
+      hipLaunchKernelGGL((attn_combine_kernel<4, false>), grid, dim3(4 * 64), 0, st, p);
+  }
   return hipGetLastError();
 }
 
@@ -1171,17 +1184,38 @@ static int attn_chunk(int seqlen_k, int splits) {
 }
 
 // Splits that follow the lengths (AttnSeq): where the split count is this
-// library's choice, there are lengths to follow and more than one split.
-static int attn_balanced(const AttnParams& p, int num_splits) {
-  return num_splits == 0 && p.seqlens && p.splits > 1 && p.batch > 1;
+// library's choice, there are lengths to follow and more than one split, and the
+// equal ones have at least `least` tokens (0: never).  The plan costs up to 1 us a
+// call, in the kernel's start and in the merge, and what it gives grows with the
+// tokens of a split.  Lengths spread evenly up to T, 64 / 8 heads, equal splits and
+// these: head-major 12.6 and 13.7 us with splits of 128 tokens (B = 4, T = 1000),
+// 20.1 and 19.3 with 256 (16 x 1000; 21.0 and 21.8 when all are T long), 29.1 and
+// 22.6 with 336 (16 x 2000); token-major 14.7 and 15.5 with 32 (4 x 256), 26.0 and
+// 22.4 with 64 (32 x 500; 26.2 and 27.0 when all are T long), 57.0 and 39.4 with
+// 256 (16 x 4000), where two splits a sequence leave little to deal out: 41.3 and
+// 46.4 with 64 (192 x 128), 63.4 and 52.7 with 256 (128 x 500).  The dense modes,
+// which stream twice as fast, keep equal splits: 64.7 and 72.1 (128 x 1000), 29.3
+// and 27.8 (8 x 4000).
+static int attn_balanced(const AttnParams& p, int num_splits, int least) {
+  return num_splits == 0 && p.seqlens && p.splits > 1 && p.batch > 1 && p.batch <= kPlanSeqs &&
+         least > 0 && p.chunk >= least;
+}
+constexpr int kBalancedFrom = 320;                             // head-major modes
+constexpr int kTmBalancedFrom = 64, kTmBalancedTwoFrom = 256;  // token-major; two splits
+
+static void attn_set_pieces(AttnParams& p, int pieces) {
+  if (!p.balanced) return;
+  p.pieces = FastDiv::of(pieces);
+  p.spare = FastDiv::of(pieces - p.batch);
 }
 
 // The splits of a call: num_splits of them, or this library's choice `own`.
-static void attn_set_splits(AttnParams& p, int num_splits, AttnSplit own) {
+static void attn_set_splits(AttnParams& p, int num_splits, AttnSplit own, int balanced_from) {
   const int steps = std::max(1, (p.seqlen_k + 15) / 16);
   p.splits = std::max(1, std::min(num_splits > 0 ? num_splits : own.splits, steps));
   p.chunk = attn_chunk(std::max(p.seqlen_k, 1), p.splits);
-  p.balanced = attn_balanced(p, num_splits);
+  p.balanced = attn_balanced(p, num_splits, balanced_from);
+  attn_set_pieces(p, p.batch * p.splits);
   p.shared = p.chunk > 64 &&
              (num_splits > 0 ? (int64_t)p.batch * p.heads_k * p.splits < kSharedItemsBelow
                              : own.shared);
@@ -1192,21 +1226,40 @@ static size_t attn_ws_bytes(int batch, int heads, int splits) {
   return (size_t)batch * heads * splits * (kHeadDim + 2) * sizeof(float);
 }
 
+// The partial results in the workspace, and behind them the plan of balanced
+// splits (without the room for it: equal splits).
+static bool attn_set_workspace(AttnParams& p, void* workspace, size_t ws_bytes) {
+  if (p.splits <= 1) return true;
+  const size_t part = attn_ws_bytes(p.batch, p.heads, p.splits);
+  if (!workspace || ws_bytes < part) return false;
+  p.ws_o = reinterpret_cast<float*>(workspace);
+  p.ws_ml = p.ws_o + (size_t)p.batch * p.heads * p.splits * kHeadDim;
+  p.plan = reinterpret_cast<int2*>(static_cast<uint8_t*>(workspace) + part);
+  if (ws_bytes < part + p.batch * sizeof(int2)) p.balanced = 0;
+  return true;
+}
+
 template <int kMode>
 static int attn_launch(hipStream_t st, AttnParams& p, void* workspace, size_t ws_bytes) {
-  if (p.splits > 1) {
-    if (!workspace || ws_bytes < attn_ws_bytes(p.batch, p.heads, p.splits)) return ZS_E_INVAL;
-    p.ws_o = reinterpret_cast<float*>(workspace);
-    p.ws_ml = p.ws_o + (size_t)p.batch * p.heads * p.splits * kHeadDim;
-  }
+  if (!attn_set_workspace(p, workspace, ws_bytes)) return ZS_E_INVAL;
   const int items = p.batch * p.heads_k * p.splits;
-  if (p.shared) {
-    // four waves per item
-    hipLaunchKernelGGL((attn_kernel<kMode, kItemWaves>), dim3(items), dim3(kItemWaves * 64), 0, st,
-                       p);
+  auto launch = [&](auto balanced) {
+    constexpr bool kBal = decltype(balanced)::value;
+    if (p.shared) {  // four waves per item
+      hipLaunchKernelGGL((attn_kernel<kMode, kItemWaves, kBal>), dim3(items), dim3(kItemWaves * 64), 0,
+                         st, p);
+    } else {
+      const int grid = (items + kAttnWaves - 1) / kAttnWaves;
+      hipLaunchKernelGGL((attn_kernel<kMode, 1, kBal>), dim3(grid), dim3(kAttnWaves * 64), 0, st, p);
+    }
+  };
+  if constexpr (kMode == kModeRetiled || kMode == kModeCanon) {
+    if (p.balanced)
+      launch(std::true_type{});
+    else
+      launch(std::false_type{});
   } else {
-    const int grid = (items + kAttnWaves - 1) / kAttnWaves;
-    hipLaunchKernelGGL((attn_kernel<kMode, 1>), dim3(grid), dim3(kAttnWaves * 64), 0, st, p);
+    launch(std::false_type{});  // (attn_balanced)
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
@@ -1281,20 +1334,19 @@ static int tm_chunk(int seqlen_k, int splits) {
 }
 
 static int attn_tm_launch(hipStream_t st, AttnParams& p, void* workspace, size_t ws_bytes) {
-  if (p.splits > 1) {
-    if (!workspace || ws_bytes < attn_ws_bytes(p.batch, p.heads, p.splits)) return ZS_E_INVAL;
-    p.ws_o = reinterpret_cast<float*>(workspace);
-    p.ws_ml = p.ws_o + (size_t)p.batch * p.heads * p.splits * kHeadDim;
-  }
+  if (!attn_set_workspace(p, workspace, ws_bytes)) return ZS_E_INVAL;
   // Grids of at most one workgroup per CU take the ring of two steps (eight
   // records per wave in flight; two waves per SIMD leave it the registers)
   // and decode phase pairs between barriers, larger grids the ring of one
   // step at four waves per SIMD.
   const int items = p.batch * p.splits;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(items), dim3(kTmWaves * 64), 0, st, p);
+  };
   if (items <= device_cu_count())
-    hipLaunchKernelGGL(attn_tm_kernel<8>, dim3(items), dim3(kTmWaves * 64), 0, st, p);
+    launch(p.balanced ? attn_tm_kernel<8, true> : attn_tm_kernel<8, false>);
   else
-    hipLaunchKernelGGL(attn_tm_kernel<4>, dim3(items), dim3(kTmWaves * 64), 0, st, p);
+    launch(p.balanced ? attn_tm_kernel<4, true> : attn_tm_kernel<4, false>);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   if (p.splits > 1) {
@@ -1336,7 +1388,8 @@ extern "C" size_t zs_decode_attention_workspace_bytes(int batch, int num_heads, 
           : std::max(std::min(std::max(1, (seqlen_k + 127) / 128),
                               (std::max(2048, 12 * device_cu_count()) + batch - 1) / batch),
                      std::min(std::max(1, (seqlen_k + 15) / 16), (kTmItems + batch - 1) / batch));
-  return attn_ws_bytes(batch, num_heads, splits);
+  return attn_ws_bytes(batch, num_heads, splits) +
+         (num_splits == 0 && splits > 1 && batch > 1 ? batch * sizeof(int2) : 0);
 }
 
 extern "C" int64_t zs_kv_retiled_staging_bytes(int layout, int rows, int cols, int num_heads_k) {
@@ -1396,10 +1449,11 @@ extern "C" int zs_decode_attention(void* stream, const uint16_t* q, const zs_kv_
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
+  const bool staged = k->layout == ZS_LAYOUT_TOKEN_MAJOR;  // dense mode, its splits
   attn_set_splits(p, num_splits,
-                  k->layout != ZS_LAYOUT_TOKEN_MAJOR
-                      ? attn_split_canonical(batch, num_heads_k, seqlen_k)
-                      : attn_split_dense(batch, num_heads_k, seqlen_k));
+                  staged ? attn_split_dense(batch, num_heads_k, seqlen_k)
+                         : attn_split_canonical(batch, num_heads_k, seqlen_k),
+                  staged ? 0 : kBalancedFrom);
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   if (k->layout == ZS_LAYOUT_TOKEN_MAJOR) {
     const size_t sk = staging_bytes(k->layout, k->rows, k->cols);
@@ -1474,14 +1528,16 @@ extern "C" int zs_decode_attention_retiled(void* stream, const uint16_t* q,
   if (k->layout == ZS_LAYOUT_TOKEN_MAJOR && tm_fused(num_heads_k, k->cols)) {
     p.splits = tm_splits(batch, seqlen_k, num_splits);
     p.chunk = tm_chunk(seqlen_k, p.splits);
-    p.balanced = attn_balanced(p, num_splits);
+    p.balanced = attn_balanced(p, num_splits, p.splits > 2 ? kTmBalancedFrom : kTmBalancedTwoFrom);
+    // (one round of them: a few more would be a second)
+    attn_set_pieces(p, std::min(p.batch * p.splits, std::max(kTmItems, batch + 1)));
     return attn_tm_launch((hipStream_t)stream, p, workspace, workspace_bytes);
   }
-  // (a staged cache runs in the dense mode, with its splits)
+  const bool staged = k->layout == ZS_LAYOUT_TOKEN_MAJOR;  // dense mode, its splits
   attn_set_splits(p, num_splits,
-                  k->layout != ZS_LAYOUT_TOKEN_MAJOR
-                      ? attn_split_retiled(batch, num_heads_k, seqlen_k)
-                      : attn_split_dense(batch, num_heads_k, seqlen_k));
+                  staged ? attn_split_dense(batch, num_heads_k, seqlen_k)
+                         : attn_split_retiled(batch, num_heads_k, seqlen_k),
+                  staged ? 0 : kBalancedFrom);
   if (k->layout == ZS_LAYOUT_TOKEN_MAJOR) {
     const size_t sk = staging_bytes(k->layout, k->rows, k->cols);
     const size_t sv = staging_bytes(v->layout, v->rows, v->cols);
@@ -1527,7 +1583,8 @@ extern "C" int zs_decode_attention_dense(void* stream, const uint16_t* q, const 
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
-  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k));
+  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k),
+                  0);
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   return attn_launch<kModeDense>((hipStream_t)stream, p, workspace, workspace_bytes);
 }
@@ -1561,7 +1618,8 @@ extern "C" int zs_decode_attention_dense_paged(
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
-  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k));
+  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k),
+                  0);
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   return attn_launch<kModePaged>((hipStream_t)stream, p, workspace, workspace_bytes);
 }

@@ -86,6 +86,20 @@ __device__ __forceinline__ void build_decode_tables(DecodeTables& T, int start_e
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// n / d for n < 2^31 by one multiply: m = ceil(2^32 / d) makes mulhi(n, m) the
+// quotient or one more.
+struct FastDiv {
+  uint32_t d, m;  // m == 0: d == 1
+  __host__ __device__ static FastDiv of(uint32_t d) {
+    return FastDiv{d, d == 1 ? 0u : 0xFFFFFFFFu / d + 1};
+  }
+  __device__ __forceinline__ uint32_t div(uint32_t n) const {
+    if (m == 0) return n;
+    const uint32_t q = __umulhi(n, m);
+    return q * d > n ? q - 1 : q;
+  }
+};
+
 // Inclusive prefix sum over the 64 lanes of a wave: Hillis-Steele inside
 // each 16-lane DPP row (row_shr 1,2,4,8), then row_bcast:15 adds row 0's
 // total into row 1 and row 2's into row 3, and row_bcast:31 adds the total of

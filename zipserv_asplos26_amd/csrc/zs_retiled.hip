@@ -39,17 +39,6 @@ struct MatSrc {
   }
 };
 
-// n / d for n < 2^31 and d >= 2 by one multiply: m = ceil(2^32 / d) makes
-// mulhi(n, m) the quotient or one more.
-struct FastDiv {
-  uint32_t d, m;  // m == 0: d == 1
-  __device__ __forceinline__ uint32_t div(uint32_t n) const {
-    if (m == 0) return n;
-    const uint32_t q = __umulhi(n, m);
-    return q * d > n ? q - 1 : q;
-  }
-};
-
 // KvSrc: a dense cache [B][T][H][D] read as the matrix that its compressed
 // form stands for -- groups of group_rows rows (head-major: one (b, h) each,
 // token-major: one b), the first `valid` rows of a group from the cache,
@@ -2455,11 +2444,8 @@ static int kv_src(const uint16_t* x, int layout, int batch, int tokens, int head
   const int64_t rows = (int64_t)batch * (hm ? heads : 1) * group_rows;
   if (group_rows < valid) return ZS_E_INVAL;
   if (rows > INT32_MAX) return ZS_E_OVERFLOW;
-  auto fast = [](uint32_t d) {
-    return FastDiv{d, d == 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1) / d)};
-  };
   const int64_t token = (int64_t)heads * head_dim;
-  *src = KvSrc{x, fast(group_rows / 16), fast(hm ? heads : 1), tokens * token, head_dim,
+  *src = KvSrc{x, FastDiv::of(group_rows / 16), FastDiv::of(hm ? heads : 1), tokens * token, head_dim,
                hm ? token : head_dim, (int)valid};
   *M = (int)rows;
   return ZS_OK;
