@@ -42,6 +42,13 @@ CASES = [
     ("token_major", 128, 128, 8, 64, True, 2),
     ("by_kv_head", 257, 1500, 1, 8, True, 2),
     ("dense", 8, 4000, 8, 64, True, 4),
+    # one wave an item where a round of shared ones is mostly start-up
+    ("by_kv_head", 256, 128, 8, 64, False, 1),
+    ("by_kv_head", 384, 128, 8, 64, False, 1),
+    ("by_kv_head", 384, 300, 8, 64, True, 1),
+    # no more splits than leave 64 tokens a wave
+    ("by_kv_head", 8, 1500, 8, 64, False, 8),
+    ("by_kv_head", 2, 6000, 8, 64, False, 32),
 ]
 
 
@@ -52,7 +59,7 @@ def test_automatic_splits_are_the_explicit_count(torch_cuda, layout, B, T, Hkv, 
         pytest.skip("the counts are those of 256 CUs")
     q, kv, lens = _inputs(torch, layout, B, T, Hkv, H, spread)
     auto, same = (_call(layout, q, kv, Hkv, T, lens, n) for n in (0, count))
-    other = _call(layout, q, kv, Hkv, T, lens, count + 1)
+    other = _call(layout, q, kv, Hkv, T, lens, 2 * count)
     torch.cuda.synchronize()
     assert torch.equal(auto.view(torch.int16), same.view(torch.int16))
     assert not torch.equal(auto.view(torch.int16), other.view(torch.int16))

@@ -1144,7 +1144,15 @@ struct AttnSplit {
   int splits;
   bool shared;
 };
-static AttnSplit attn_split_retiled(int batch, int heads_k, int seqlen_k) {
+//
+// Where both would leave the sequences whole, no merge is saved and a round of
+// shared items pays its start-up (kStart tokens of one wave) for a quarter of the
+// tokens; a round of one-wave items that fills a share r of the places costs
+// max(0.4, r + 0.08) of a full one, or r where shorter sequences make room.  B =
+// 384, T = 128: 32.0 us with one wave an item, 48.9 shared; B = 264, T = 800:
+// 152.5 and 132.9 (8 KV heads; 17 batches of 200..1000 by 9 lengths of 64..1000,
+// both timed at each: the choice is at most 4% off).
+static AttnSplit attn_split_retiled(int batch, int heads_k, int seqlen_k, bool lengths) {
   const int64_t units = std::max<int64_t>(1, (int64_t)batch * heads_k);
   const int64_t slots = 3 * (int64_t)device_cu_count();
   auto pick = [&](int64_t slots, int min_tokens, int64_t most) {
@@ -1156,8 +1164,22 @@ static AttnSplit attn_split_retiled(int batch, int heads_k, int seqlen_k) {
     return (double)items / ((items + slots - 1) / slots * slots);
   };
   const int64_t sh = pick(slots, 128, 64), one = pick(slots * kAttnWaves, 256, INT32_MAX);
+  if (one == 1 && 3 * units >= 2 * slots * kAttnWaves) {
+    constexpr double kStart = 19;
+    const double rs = (double)units / slots, ro = rs / kAttnWaves;
+    const double full = std::floor(ro), part = std::min(1., ro - full + 0.08);
+    const double busy = lengths && ro >= 1 ? ro : full + (ro > full ? std::max(0.4, part) : 0.);
+    return {1, kStart * std::ceil(rs) + seqlen_k * rs / kAttnWaves <
+                   kStart * std::ceil(ro) + seqlen_k * busy};
+  }
   const double fs = filled(sh * units, slots), fo = filled(one * units, slots * kAttnWaves);
-  if (fs >= 0.9 * fo) return {(int)sh, true};
+  if (fs >= 0.9 * fo) {
+    // (under 64 tokens a wave the merge costs more than the fuller round gives: B = 2, T =
+    // 6000 18.0 us with 32 splits, 18.8 with 47; B = 8, T = 1500 18.1 with 8, 19.0 with 12)
+    const bool small = seqlen_k < 256 * sh;
+    return {small ? std::min((int)sh, attn_auto_splits(batch, heads_k, seqlen_k, true)) : (int)sh,
+            true};
+  }
   return {(int)one, false};
 }
 
@@ -1169,10 +1191,10 @@ static AttnSplit attn_split_canonical(int batch, int heads_k, int seqlen_k) {
 
 // Splits of the dense modes: on large grids the re-tiled mode's, so that the
 // two walk the same pieces, else attn_auto_splits.
-static AttnSplit attn_split_dense(int batch, int heads_k, int seqlen_k) {
+static AttnSplit attn_split_dense(int batch, int heads_k, int seqlen_k, bool lengths) {
   const int s = attn_auto_splits(batch, heads_k, seqlen_k, false);
   if ((int64_t)s * batch * heads_k >= kSharedItemsBelow)
-    return attn_split_retiled(batch, heads_k, seqlen_k);
+    return attn_split_retiled(batch, heads_k, seqlen_k, lengths);
   return {s, true};
 }
 
@@ -1451,7 +1473,7 @@ extern "C" int zs_decode_attention(void* stream, const uint16_t* q, const zs_kv_
   p.group = num_heads / num_heads_k;
   const bool staged = k->layout == ZS_LAYOUT_TOKEN_MAJOR;  // dense mode, its splits
   attn_set_splits(p, num_splits,
-                  staged ? attn_split_dense(batch, num_heads_k, seqlen_k)
+                  staged ? attn_split_dense(batch, num_heads_k, seqlen_k, cache_seqlens)
                          : attn_split_canonical(batch, num_heads_k, seqlen_k),
                   staged ? 0 : kBalancedFrom);
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
@@ -1535,8 +1557,8 @@ extern "C" int zs_decode_attention_retiled(void* stream, const uint16_t* q,
   }
   const bool staged = k->layout == ZS_LAYOUT_TOKEN_MAJOR;  // dense mode, its splits
   attn_set_splits(p, num_splits,
-                  staged ? attn_split_dense(batch, num_heads_k, seqlen_k)
-                         : attn_split_retiled(batch, num_heads_k, seqlen_k),
+                  staged ? attn_split_dense(batch, num_heads_k, seqlen_k, cache_seqlens)
+                         : attn_split_retiled(batch, num_heads_k, seqlen_k, cache_seqlens),
                   staged ? 0 : kBalancedFrom);
   if (k->layout == ZS_LAYOUT_TOKEN_MAJOR) {
     const size_t sk = staging_bytes(k->layout, k->rows, k->cols);
@@ -1583,7 +1605,7 @@ extern "C" int zs_decode_attention_dense(void* stream, const uint16_t* q, const 
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
-  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k),
+  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k, cache_seqlens),
                   0);
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   return attn_launch<kModeDense>((hipStream_t)stream, p, workspace, workspace_bytes);
@@ -1618,7 +1640,7 @@ extern "C" int zs_decode_attention_dense_paged(
   p.heads = num_heads;
   p.heads_k = num_heads_k;
   p.group = num_heads / num_heads_k;
-  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k),
+  attn_set_splits(p, num_splits, attn_split_dense(batch, num_heads_k, seqlen_k, cache_seqlens),
                   0);
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   return attn_launch<kModePaged>((hipStream_t)stream, p, workspace, workspace_bytes);
