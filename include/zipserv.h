@@ -47,6 +47,7 @@ extern "C" {
 #define ZS_STREAM_SLACK_BYTES 64
 /* Bytes of d_tmp per 16 x 64 record for zs_compress_retiled_fixed_gpu. */
 #define ZS_RETILED_EXP_SLOT_BYTES 256
+#define ZS_RETILED_WHOLE_SLOT_BYTES 1024 /* a record's elements: every one an outlier */
 /* Window rules of zs_compress_retiled_auto_gpu: the KV-cache compressor's
  * (zipserv_decode_attention_ext.cu:65-134) and the weight path's
  * (kernel_benchmark/utils.h:189-272). */
@@ -253,7 +254,7 @@ int zs_compress_retiled_exps_gpu(void* stream, const uint16_t* d_input, int M, i
  * head) (ZS_LAYOUT_HEAD_MAJOR, >= tokens) or per batch entry
  * (ZS_LAYOUT_TOKEN_MAJOR, >= tokens * heads), a multiple of 16, the rows past
  * the cache's own zero.  The bytes are those of the padded matrix; no copy of
- * the cache is made. */
+ * the cache is made, so it must stay as it is until the second one has run. */
 int zs_compress_retiled_kv_gpu(void* stream, const uint16_t* d_cache, int layout, int batch,
                                int tokens, int heads, int head_dim, int group_rows, int rule,
                                uint64_t* d_hist, int32_t* d_top, uint8_t* d_work,
@@ -263,6 +264,17 @@ int zs_compress_retiled_kv_exps_gpu(void* stream, const uint16_t* d_cache, int l
                                     int tokens, int heads, int head_dim, int group_rows,
                                     const int32_t* d_top_exponents, const int32_t* d_eoff,
                                     const uint8_t* d_tmp, uint8_t* d_exps);
+/* The same with slots of ZS_RETILED_WHOLE_SLOT_BYTES in d_tmp, which hold every
+ * record's outlier bytes: the cache is read by the first call alone, which takes a
+ * snapshot of it in stream order, and the second one takes the M x K of the padded
+ * matrix. */
+int zs_compress_retiled_kv_whole_gpu(void* stream, const uint16_t* d_cache, int layout, int batch,
+                                     int tokens, int heads, int head_dim, int group_rows, int rule,
+                                     uint64_t* d_hist, int32_t* d_top, uint8_t* d_work,
+                                     uint8_t* d_fixed, int32_t* d_counts, int32_t* d_eoff,
+                                     int64_t* d_total, uint8_t* d_tmp);
+int zs_compress_retiled_whole_exps_gpu(void* stream, int M, int K, const int32_t* d_eoff,
+                                       const uint8_t* d_tmp, uint8_t* d_exps);
 /* Canonical TCA-TBE streams -> re-tiled, same two phases (window start_exp). */
 int zs_retile_triple_bitmap_count_gpu(void* stream, const uint8_t* SignMantissa,
                                       const uint16_t* CompressedFull, const uint64_t* Bitmap1,

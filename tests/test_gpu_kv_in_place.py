@@ -56,6 +56,60 @@ def test_in_place_outliers_past_the_slot(torch_cuda, layout):
     _compare(to_torch_bf16(a), layout)
 
 
+@pytest.mark.parametrize("layout", ["by_kv_head", "token_major"])
+@pytest.mark.parametrize("noise", [False, True])
+def test_the_cache_may_change_once_it_is_encoded(torch_cuda, layout, noise):
+    # what is written into the cache behind the first phase, by another thread
+    # or after the call returned, is not in the stream: also for records with
+    # more outliers than an ordinary slot holds (rows of random bits; the band
+    # where a sequence ends)
+    import zipserv_asplos26_amd as zs
+    import zipserv_asplos26_amd.attention as za
+    from zipserv_asplos26_amd import codec
+    rng = np.random.default_rng(6)
+    a = kv_bf16(rng, 2, 301, 8, 128)
+    if noise:
+        a[:, 40:140] = rng.integers(0, 1 << 16, a[:, 40:140].shape, dtype=np.uint16)
+    x = to_torch_bf16(a)
+    m, logical, _ = _matrix(za, x, layout, 16)
+    want = zs.compress_retiled(m.contiguous(), logical, 128, layout=layout)
+    group, _ = za._kv_group(x, layout, 16)
+    lid = za.LAYOUT_IDS[layout]
+    s = codec._retiled_encode(x, "kv", kv=(lid, *x.shape, group))
+    x.copy_(to_torch_bf16(rng.integers(0, 1 << 16, x.shape, dtype=np.uint16)))
+    _same(codec._retiled_finish(s, s["meta"].cpu(), logical, 128, layout), want)
+
+
+@pytest.mark.parametrize("layout", ["by_kv_head", "token_major"])
+def test_in_place_bytes_with_ordinary_slots(torch_cuda, layout):
+    # zs_compress_retiled_kv_gpu / _kv_exps_gpu, whose second call reads the
+    # records past their slots from the cache again
+    import zipserv_asplos26_amd as zs
+    import zipserv_asplos26_amd.attention as za
+    torch, L = torch_cuda, zs.lib()
+    rng = np.random.default_rng(7)
+    a = kv_bf16(rng, 2, 301, 8, 128)
+    a[:, 40:140] = rng.integers(0, 1 << 16, a[:, 40:140].shape, dtype=np.uint16)
+    x = to_torch_bf16(a)
+    want = za.compress_kv(x, layout, retiled=True)
+    shape = (za.LAYOUT_IDS[layout], *x.shape, za._kv_group(x, layout, 16)[0])
+    n = want.rows // 16 * (want.cols // 64)
+    new = lambda k, dtype: torch.empty(k, dtype=dtype, device="cuda")
+    hist, top, work = new(256, torch.int64), new(7, torch.int32), new(
+        zs._lib.ZS_RETILED_AUTO_WORK_BYTES, torch.uint8)
+    fixed, cnt, eoff = new(n * 1408, torch.uint8), new(n, torch.int32), new(n + 1, torch.int32)
+    total, tmp, exps = new(1, torch.int64), new(n * 256, torch.uint8), torch.empty_like(want.exps)
+    st = int(torch.cuda.current_stream().cuda_stream)
+    ptrs = [t.data_ptr() for t in (hist, top, work, fixed, cnt, eoff, total, tmp)]
+    assert L.zs_compress_retiled_kv_gpu(st, x.data_ptr(), *shape, zs._lib.ZS_WINDOW_KV, *ptrs) == 0
+    assert int(total) == want.num_outliers
+    assert L.zs_compress_retiled_kv_exps_gpu(st, x.data_ptr(), *shape, top.data_ptr(),
+                                             eoff.data_ptr(), tmp.data_ptr(), exps.data_ptr()) == 0
+    torch.cuda.synchronize()
+    for got, ref in ((fixed, want.fixed), (eoff, want.eoff), (exps, want.exps)):
+        assert torch.equal(got, ref)
+
+
 @pytest.mark.parametrize("T", [65, 4097])
 def test_in_place_zero_padding_moves_the_window(torch_cuda, T):
     # one or two distinct exponents and much padding: the padding's zeros are

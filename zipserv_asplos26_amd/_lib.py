@@ -20,6 +20,7 @@ ZS_E_OVERFLOW = -3
 ZS_E_NOMEM = -4
 ZS_STREAM_SLACK_BYTES = 64
 ZS_RETILED_EXP_SLOT_BYTES = 256
+ZS_RETILED_WHOLE_SLOT_BYTES = 1024
 ZS_WINDOW_KV = 0
 ZS_WINDOW_WEIGHTS = 1
 ZS_RETILED_AUTO_WORK_BYTES = 65600
@@ -72,6 +73,8 @@ SIGNATURES = {
     "zs_compress_retiled_exps_gpu": (C.c_int, [_p, _p, C.c_int, C.c_int, _p, _p, _p, _p]),
     "zs_compress_retiled_kv_gpu": (C.c_int, [_p, _p] + [C.c_int] * 7 + [_p] * 8),
     "zs_compress_retiled_kv_exps_gpu": (C.c_int, [_p, _p] + [C.c_int] * 6 + [_p] * 4),
+    "zs_compress_retiled_kv_whole_gpu": (C.c_int, [_p, _p] + [C.c_int] * 7 + [_p] * 8),
+    "zs_compress_retiled_whole_exps_gpu": (C.c_int, [_p, C.c_int, C.c_int, _p, _p, _p]),
     "zs_retile_triple_bitmap_count_gpu": (
         C.c_int, [_p, _p, _p, _p, _p, _p, _p, _p, C.c_int, C.c_int, _p, _p, _p]),
     "zs_retile_triple_bitmap_emit_gpu": (

@@ -507,9 +507,10 @@ def _retiled_encode(input, window, guess=None, kv=None):
     exponent stream.  Under a window rule, `guess` (int32 [7] on the device,
     e.g. the previous matrix's window) replaces the sampled guess; the bytes
     are the same either way.  `kv` (layout id, batch, tokens, heads, head_dim,
-    group_rows; zs_compress_retiled_kv_gpu): `input` is a dense cache, encoded
-    as the padded matrix of that layout.  Returns the state _retiled_finish
-    takes."""
+    group_rows; zs_compress_retiled_kv_whole_gpu): `input` is a dense cache,
+    encoded as the padded matrix of that layout and not read again by the second
+    phase, so that the caller may change or free it once this phase has run.
+    Returns the state _retiled_finish takes."""
     torch = _torch()
     _check_cuda(input, "input", torch.bfloat16)
     if kv is not None:
@@ -531,7 +532,8 @@ def _retiled_encode(input, window, guess=None, kv=None):
     counts = torch.empty(256, dtype=torch.int64, device=dev)
     cnt, eoff = torch.empty(nrec, **i32), torch.empty(nrec + 1, **i32)
     fixed = torch.empty(nrec * 1408, dtype=torch.uint8, device=dev)
-    tmp = torch.empty(nrec * _lib.ZS_RETILED_EXP_SLOT_BYTES, dtype=torch.uint8, device=dev)
+    slot = _lib.ZS_RETILED_EXP_SLOT_BYTES if kv is None else _lib.ZS_RETILED_WHOLE_SLOT_BYTES
+    tmp = torch.empty(nrec * slot, dtype=torch.uint8, device=dev)
     st = _stream()
     if isinstance(window, str):
         if window not in WINDOW_RULES:
@@ -540,10 +542,11 @@ def _retiled_encode(input, window, guess=None, kv=None):
         work = torch.empty(_lib.ZS_RETILED_AUTO_WORK_BYTES, dtype=torch.uint8, device=dev)
         # 64-bit bins: the re-tiled layout takes matrices past 2^31 elements.
         if kv is not None:
-            check("zs_compress_retiled_kv_gpu",
-                  L.zs_compress_retiled_kv_gpu(st, _dptr(input), *kv, rule, _dptr(counts),
-                                               _dptr(top), _dptr(work), _dptr(fixed), _dptr(cnt),
-                                               _dptr(eoff), _dptr(total), _dptr(tmp)))
+            check("zs_compress_retiled_kv_whole_gpu",
+                  L.zs_compress_retiled_kv_whole_gpu(st, _dptr(input), *kv, rule, _dptr(counts),
+                                                     _dptr(top), _dptr(work), _dptr(fixed),
+                                                     _dptr(cnt), _dptr(eoff), _dptr(total),
+                                                     _dptr(tmp)))
         elif guess is not None:
             _check_cuda(guess, "guess", torch.int32)
             check("zs_compress_retiled_guess_gpu",
@@ -577,13 +580,15 @@ def _retiled_finish(s, host_meta, logical_rows, logical_cols, layout) -> Zipserv
     # every byte is written by the compaction, the slack bytes as zeros
     exps = torch.empty(tot + _lib.ZS_STREAM_SLACK_BYTES, dtype=torch.uint8,
                        device=s["input"].device)
-    args = [_dptr(s["top"]), _dptr(s["eoff"]), _dptr(s["tmp"]), _dptr(exps)]
     if s["kv"] is not None:
-        check("zs_compress_retiled_kv_exps_gpu",
-              lib().zs_compress_retiled_kv_exps_gpu(_stream(), _dptr(s["input"]), *s["kv"], *args))
+        check("zs_compress_retiled_whole_exps_gpu",
+              lib().zs_compress_retiled_whole_exps_gpu(_stream(), rows, cols, _dptr(s["eoff"]),
+                                                       _dptr(s["tmp"]), _dptr(exps)))
     else:
         check("zs_compress_retiled_exps_gpu",
-              lib().zs_compress_retiled_exps_gpu(_stream(), _dptr(s["input"]), rows, cols, *args))
+              lib().zs_compress_retiled_exps_gpu(_stream(), _dptr(s["input"]), rows, cols,
+                                                 _dptr(s["top"]), _dptr(s["eoff"]), _dptr(s["tmp"]),
+                                                 _dptr(exps)))
     s.pop("tmp")  # stream-ordered: the allocator reuses it only after the compaction
     return ZipservRetiled(s["fixed"], exps, s["eoff"], rows, cols,
                           rows if logical_rows is None else logical_rows,
@@ -610,8 +615,10 @@ def compress_retiled_kv(cache, layout: str, group_rows: int, logical_rows: int) 
     """compress_retiled of a contiguous dense cache (batch, tokens, heads,
     head_dim) as the padded matrix of `layout` ("by_kv_head", or a token-major
     one), which is not built: the encoder reads the cache in that order
-    (zs_compress_retiled_kv_gpu).  group_rows: the matrix's rows per (batch,
-    head), or per batch entry."""
+    (zs_compress_retiled_kv_whole_gpu).  The result is a snapshot of the cache in
+    stream order, and every read of it has ended on return: the outlier slots
+    hold whole records (half the cache's bytes while the call runs).  group_rows: the
+    matrix's rows per (batch, head), or per batch entry."""
     B, T, H, D = cache.shape
     lid = _lib.ZS_LAYOUT_HEAD_MAJOR if layout == "by_kv_head" else _lib.ZS_LAYOUT_TOKEN_MAJOR
     s = _retiled_encode(cache, "kv", kv=(lid, B, T, H, D, group_rows))

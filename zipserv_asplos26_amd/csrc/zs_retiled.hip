@@ -29,9 +29,13 @@ __device__ __forceinline__ const uint16_t* rec_src_at(const uint16_t* a, int K, 
   return a + (band * 16 + (l & 15)) * (int64_t)K + kt * 64 + 32 * h + 8 * (l >> 4);
 }
 
+constexpr int kExpSlot = ZS_RETILED_EXP_SLOT_BYTES;
+
 // Where the encoders read a record's 16 x 64 elements: lane l's eight of half
-// h of the tile (band, kt).  MatSrc: a row-major matrix.
+// h of the tile (band, kt); kSlot: bytes of a record's outlier slot.  MatSrc: a
+// row-major matrix.
 struct MatSrc {
+  static constexpr int kSlot = kExpSlot;
   const uint16_t* a;
   int K;
   __device__ __forceinline__ u32x4 load(int64_t band, int kt, int h) const {
@@ -45,6 +49,7 @@ struct MatSrc {
 // the rest zeros -- so that no padded, transposed copy is written and read
 // back first.  16-row bands do not cross groups (group_rows % 16 == 0).
 struct KvSrc {
+  static constexpr int kSlot = kExpSlot;
   const uint16_t* x;
   FastDiv bands, inner;  // bands per group; groups per batch (head-major: H)
   int64_t outer_stride, inner_stride, row_stride;  // elements
@@ -58,6 +63,13 @@ struct KvSrc {
                                                     8 * (lane_id() >> 4));
     return r < valid ? v : u32x4{0, 0, 0, 0};
   }
+};
+
+// KvSrc with slots that hold every record: the cache is read by the encoding pass
+// alone, so that the stream is a snapshot of it.
+struct KvWholeSrc : KvSrc {
+  static constexpr int kSlot = ZS_RETILED_WHOLE_SLOT_BYTES;
+  __host__ __device__ explicit KvWholeSrc(const KvSrc& s) : KvSrc(s) {}
 };
 
 // The records a wave of a grid-stride loop visits -- rec = w, w + nw, ...
@@ -425,8 +437,6 @@ __device__ __forceinline__ RecCodes rec_codes(const u32x4 v[2], uint32_t st) {
 // Element of bit 3i of z (i = 3i / 3 for 3i <= 21).
 __device__ __forceinline__ int rec_elem(int bit3) { return (bit3 * 11) >> 5; }
 
-constexpr int kExpSlot = ZS_RETILED_EXP_SLOT_BYTES;
-
 // Exponents of a half's eight elements, a byte each (of a dword rotated left by
 // one bit, the exponents are bytes 1 and 3).
 __device__ __forceinline__ void rec_exps(const u32x4& v, uint32_t (&e)[2]) {
@@ -469,13 +479,13 @@ __device__ __forceinline__ void outlier_exps(uint8_t* o0, uint8_t* o1, uint32_t*
 }
 
 // emit_record from rec_codes: the fixed part, and the outlier bytes to the
-// record's slot (kExpSlot bytes, 4-byte aligned) unless there are more of
+// record's slot (kSlot bytes, 4-byte aligned) unless there are more of
 // them than it holds; they are put together in `lds` (1024 bytes of this wave)
-// and stored as one dword per lane.  One walk over the outliers for bytes and
+// and stored by the dword.  One walk over the outliers for bytes and
 // histogram instead of one each over the input dwords: a cache of 258048 x 128
 // elements with 10% outliers 35.1 -> 31.0 us, 14336 x 4096 with 3% 44.8 -> 41.6.  Returns
 // the record's outlier count.
-template <bool kHist>
+template <bool kHist, int kSlot>
 __device__ __forceinline__ int emit_record_c(uint8_t* fixed, uint8_t* slot, uint8_t* lds,
                                              uint32_t* bins, int64_t rec, const u32x4 v[2],
                                              const RecCodes& rc) {
@@ -500,8 +510,13 @@ __device__ __forceinline__ int emit_record_c(uint8_t* fixed, uint8_t* slot, uint
   r_scan(n0, n1, rank0, rank1);
   const int total = __builtin_amdgcn_readlane(rank1 + (int)n1, 63);
   outlier_exps<kHist>(lds + rank0, lds + rank1, bins, e, rc.z);
-  if (total <= kExpSlot && 4 * l < total)
-    reinterpret_cast<uint32_t*>(slot)[l] = reinterpret_cast<const uint32_t*>(lds)[l];
+  if (total <= kSlot) {
+#pragma unroll
+    for (int d0 = 0; d0 < kSlot; d0 += 256)
+      if (d0 + 4 * l < total)
+        *reinterpret_cast<uint32_t*>(slot + d0 + 4 * l) =
+            *reinterpret_cast<const uint32_t*>(lds + d0 + 4 * l);
+  }
   return total;
 }
 
@@ -598,7 +613,7 @@ __global__ __launch_bounds__(256) void rfixed_kernel(Src src, int M, int K,
         cc[c - 1] += __builtin_popcount((c & 1 ? P[0] : ~P[0]) & (c & 2 ? P[1] : ~P[1]) &
                                         (c & 4 ? P[2] : ~P[2]) & 0x6DB6DBu);
     }
-    const int n = emit_record_c<kHist>(fixed, tmp + rec * kExpSlot, xb, lh, rec, v, rc);
+    const int n = emit_record_c<kHist, Src::kSlot>(fixed, tmp + rec * Src::kSlot, xb, lh, rec, v, rc);
     if (lane_id() == 0) counts[rec] = n;
   }
   if constexpr (kHist) {
@@ -623,7 +638,7 @@ __global__ __launch_bounds__(256) void rfixed_kernel(Src src, int M, int K,
 // first and last dwords -- shared with the neighbouring records -- byte by
 // byte.  Only the slot dwords that hold outlier bytes are read.  A record
 // with more outlier bytes than its slot holds is emitted from a re-read of
-// its input tile.  With n <= kExpSlot - 4 the lanes that write stay below
+// its input tile, one past the first 256 bytes of a whole slot from the slot.  With n <= kExpSlot - 4 the lanes that write stay below
 // (n + 3 + 3) / 4 <= kExpSlot / 4, so slot dword l (and l - 1) is in range.
 // Few records per wave keep each wave's chain of dependent memory operations
 // short; the grid, not the wave, supplies the parallelism.
@@ -660,7 +675,8 @@ __global__ __launch_bounds__(256) void rcompact_kernel(Src src, int M, int K,
                                                        uint8_t* __restrict__ exps) {
   __shared__ __attribute__((aligned(16))) uint8_t cbuf[4 * kCompactBuf];
   uint8_t* buf = cbuf + (threadIdx.x >> 6) * kCompactBuf;
-  const uint32_t st = (uint32_t)(top[0] - 1) & 0xFFu;
+  constexpr bool kWhole = Src::kSlot >= 1024;  // no record is read again (top: not used)
+  const uint32_t st = kWhole ? 0u : (uint32_t)(top[0] - 1) & 0xFFu;
   const int64_t nrec = (int64_t)(M >> 4) * (K >> 6);
   // the stream's slack bytes (read past the end, never selected) as zeros
   if (blockIdx.x == 0 && threadIdx.x < ZS_STREAM_SLACK_BYTES)
@@ -677,7 +693,7 @@ __global__ __launch_bounds__(256) void rcompact_kernel(Src src, int M, int K,
 #pragma unroll
     for (int q = 0; q < kCompactRecs; ++q)
       cur[q] = q < cnt && l < kExpSlot / 4 && 4 * l < __builtin_amdgcn_readlane(nl, q) + 4
-                   ? tmp32[(r0 + q) * (kExpSlot / 4) + l]
+                   ? tmp32[(r0 + q) * (Src::kSlot / 4) + l]
                    : 0u;
 #pragma unroll
     for (int q = 0; q < kCompactRecs; ++q) prev[q] = __shfl_up(cur[q], 1);
@@ -704,7 +720,7 @@ __global__ __launch_bounds__(256) void rcompact_kernel(Src src, int M, int K,
       put_range(buf, exps, E0, E1);
       continue;
     }
-    uint32_t slow = 0;  // records re-read from the input
+    uint32_t slow = 0;  // records of more outliers than the first 256 bytes of a slot
 #pragma unroll
     for (int q = 0; q < kCompactRecs; ++q) {
       const int n = __builtin_amdgcn_readlane(nl, q);
@@ -727,6 +743,30 @@ __global__ __launch_bounds__(256) void rcompact_kernel(Src src, int M, int K,
       }
     }
     if (!slow) continue;
+    if constexpr (kWhole) {
+      while (slow) {
+        const int q = __builtin_ctz(slow);
+        slow &= slow - 1;
+        const uint32_t* slot = tmp32 + (r0 + q) * (Src::kSlot / 4);
+        const int n = __builtin_amdgcn_readlane(nl, q), e0 = __builtin_amdgcn_readlane(e0l, q);
+        const int al = e0 & 3;
+        // dword d of the stream from the record's first one on: slot bytes 4d - al
+        // .. 4d - al + 3
+        for (int d = l; 4 * d < n + al; d += 64) {
+          const uint32_t lo = d > 0 ? slot[d - 1] : 0u, hi = d < Src::kSlot / 4 ? slot[d] : 0u;
+          const uint32_t v = al == 0 ? hi : __builtin_amdgcn_alignbyte(hi, lo, 4 - al);
+          uint8_t* o = exps + (e0 - al) + 4 * (int64_t)d;
+          if (4 * d >= al && 4 * d + 4 <= n + al) {
+            *reinterpret_cast<uint32_t*>(o) = v;
+          } else {
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+              if (4 * d + b >= al && 4 * d + b < n + al) o[b] = (uint8_t)(v >> (8 * b));
+          }
+        }
+      }
+      continue;
+    }
     // each one's tile is loaded while the one before it is emitted (a padded
     // cache's rows of zeros are runs of such records, a memory latency each)
     const int KT = K >> 6;
@@ -2451,19 +2491,48 @@ static int kv_src(const uint16_t* x, int layout, int batch, int tokens, int head
   return ZS_OK;
 }
 
+template <typename Src>
+static int retiled_kv(void* stream, const uint16_t* d_cache, int layout, int batch, int tokens,
+                      int heads, int head_dim, int group_rows, int rule, uint64_t* d_hist,
+                      int32_t* d_top, uint8_t* d_work, uint8_t* d_fixed, int32_t* d_counts,
+                      int32_t* d_eoff, int64_t* d_total, uint8_t* d_tmp) {
+  KvSrc src;
+  int M;
+  const int c = kv_src(d_cache, layout, batch, tokens, heads, head_dim, group_rows, &src, &M);
+  if (c != ZS_OK) return c;
+  const int64_t n = (int64_t)batch * tokens * heads * head_dim;
+  return retiled_auto(stream, Src(src), d_cache, n, (int64_t)M * head_dim - n, M, head_dim, rule,
+                      nullptr, d_hist, d_top, d_work, d_fixed, d_counts, d_eoff, d_total, d_tmp);
+}
+
 extern "C" int zs_compress_retiled_kv_gpu(void* stream, const uint16_t* d_cache, int layout,
                                           int batch, int tokens, int heads, int head_dim,
                                           int group_rows, int rule, uint64_t* d_hist,
                                           int32_t* d_top, uint8_t* d_work, uint8_t* d_fixed,
                                           int32_t* d_counts, int32_t* d_eoff, int64_t* d_total,
                                           uint8_t* d_tmp) {
-  KvSrc src;
-  int M;
-  const int c = kv_src(d_cache, layout, batch, tokens, heads, head_dim, group_rows, &src, &M);
-  if (c != ZS_OK) return c;
-  const int64_t n = (int64_t)batch * tokens * heads * head_dim;
-  return retiled_auto(stream, src, d_cache, n, (int64_t)M * head_dim - n, M, head_dim, rule,
-                      nullptr, d_hist, d_top, d_work, d_fixed, d_counts, d_eoff, d_total, d_tmp);
+  return retiled_kv<KvSrc>(stream, d_cache, layout, batch, tokens, heads, head_dim, group_rows, rule,
+                           d_hist, d_top, d_work, d_fixed, d_counts, d_eoff, d_total, d_tmp);
+}
+
+extern "C" int zs_compress_retiled_kv_whole_gpu(void* stream, const uint16_t* d_cache, int layout,
+                                                int batch, int tokens, int heads, int head_dim,
+                                                int group_rows, int rule, uint64_t* d_hist,
+                                                int32_t* d_top, uint8_t* d_work, uint8_t* d_fixed,
+                                                int32_t* d_counts, int32_t* d_eoff,
+                                                int64_t* d_total, uint8_t* d_tmp) {
+  return retiled_kv<KvWholeSrc>(stream, d_cache, layout, batch, tokens, heads, head_dim, group_rows,
+                                rule, d_hist, d_top, d_work, d_fixed, d_counts, d_eoff, d_total,
+                                d_tmp);
+}
+
+template <typename Src>
+static int launch_compact(void* stream, const Src& src, int M, int K, const int32_t* d_top,
+                          const int32_t* d_eoff, const uint8_t* d_tmp, uint8_t* d_exps) {
+  const int64_t nrec = (int64_t)(M / 16) * (K / 64);
+  hipLaunchKernelGGL(rcompact_kernel<Src>, dim3(r_grid((nrec + kCompactRecs - 1) / kCompactRecs, 4)),
+                     dim3(256), 0, (hipStream_t)stream, src, M, K, d_top, d_eoff, d_tmp, d_exps);
+  return status_of(hipGetLastError());
 }
 
 template <typename Src>
@@ -2472,10 +2541,13 @@ static int retiled_exps(void* stream, const Src& src, const uint16_t* dense, int
                         uint8_t* d_exps) {
   if (!shape_ok(M, K) || !dense || !d_top || !d_eoff || !d_tmp || !d_exps) return ZS_E_INVAL;
   if (reinterpret_cast<uintptr_t>(dense) & 15) return ZS_E_INVAL;
-  const int64_t nrec = (int64_t)(M / 16) * (K / 64);
-  hipLaunchKernelGGL(rcompact_kernel<Src>, dim3(r_grid((nrec + kCompactRecs - 1) / kCompactRecs, 4)),
-                     dim3(256), 0, (hipStream_t)stream, src, M, K, d_top, d_eoff, d_tmp, d_exps);
-  return status_of(hipGetLastError());
+  return launch_compact(stream, src, M, K, d_top, d_eoff, d_tmp, d_exps);
+}
+
+extern "C" int zs_compress_retiled_whole_exps_gpu(void* stream, int M, int K, const int32_t* d_eoff,
+                                                  const uint8_t* d_tmp, uint8_t* d_exps) {
+  if (!shape_ok(M, K) || !d_eoff || !d_tmp || !d_exps) return ZS_E_INVAL;
+  return launch_compact(stream, KvWholeSrc(KvSrc{}), M, K, nullptr, d_eoff, d_tmp, d_exps);
 }
 
 extern "C" int zs_compress_retiled_exps_gpu(void* stream, const uint16_t* d_input, int M, int K,
