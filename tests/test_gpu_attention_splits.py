@@ -49,9 +49,6 @@ CASES = [
     # no more splits than leave 64 tokens a wave
     ("by_kv_head", 8, 1500, 8, 64, False, 8),
     ("by_kv_head", 2, 6000, 8, 64, False, 32),
-    # the dense mode's own count where items are not shared
-    ("dense", 1024, 600, 1, 8, True, 2),
-    ("dense", 128, 1000, 8, 64, True, 2),
 ]
 
 

@@ -1189,15 +1189,13 @@ static AttnSplit attn_split_canonical(int batch, int heads_k, int seqlen_k) {
   return {s, (int64_t)s * batch * heads_k < kSharedItemsBelow};
 }
 
-// Splits of the dense modes: on large grids shared items where the re-tiled mode
-// would share them (24 x 6000 tokens, 64 / 8 heads 145.6 -> 122.7 us), else attn_auto_splits
-// (more one-wave splits, as the re-tiled mode takes, lose: 1024 x up to 600, 8 / 1 heads
-// 51.1 -> 55.4).
+// Splits of the dense modes: on large grids the re-tiled mode's, so that the
+// two walk the same pieces, else attn_auto_splits.
 static AttnSplit attn_split_dense(int batch, int heads_k, int seqlen_k, bool lengths) {
   const int s = attn_auto_splits(batch, heads_k, seqlen_k, false);
-  if ((int64_t)s * batch * heads_k < kSharedItemsBelow) return {s, true};
-  const AttnSplit r = attn_split_retiled(batch, heads_k, seqlen_k, lengths);
-  return r.shared ? r : AttnSplit{s, false};
+  if ((int64_t)s * batch * heads_k >= kSharedItemsBelow)
+    return attn_split_retiled(batch, heads_k, seqlen_k, lengths);
+  return {s, true};
 }
 
 // Tokens per split: a multiple of 16 (one median, one record band), so that
