@@ -239,3 +239,34 @@ def test_canonical_zipgemm_x_past_2gib(torch_cuda, split_k):
     torch.cuda.synchronize()
     err = float((y.float() - ref).abs().max() / ref.abs().max())
     assert err < 1e-2, err
+
+
+@pytest.mark.parametrize("end", ["past their slots", "in their slots"])
+def test_outlier_stream_that_ends_just_below_2_31(torch_cuda, end):
+    # 2^31 - 100 outlier bytes, the last records with more of them than a slot
+    # holds, or few enough for the compaction's common path: the first and last
+    # rows' bytes are those of the same rows compressed alone
+    torch = torch_cuda
+    M, K, window = 524352, 4096, [120 + i for i in range(7)]
+    x = torch.zeros(M, K, dtype=torch.int16, device="cuda")  # exponent 0: outliers
+    inside = M * K - (2**31 - 100)  # elements of exponent 120
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9)
+    tail = torch.randint(0, 100, (64, K), dtype=torch.int16, device="cuda", generator=g) << 7
+    if end == "in their slots":
+        last = torch.full((16, 512), 120 << 7, dtype=torch.int16, device="cuda")
+        last.view(16, 8, 64)[:, :, :12] = tail[-16:, -512:].reshape(16, 8, 64)[:, :, :12]
+        tail[-16:, -512:] = last
+        inside -= 16 * 8 * 52
+    x[-64:] = tail
+    x.view(-1)[:inside] = 120 << 7
+    x = x.view(torch.bfloat16)
+    r = zs.compress_retiled(x, window=window)
+    torch.cuda.synchronize()
+    assert r.num_outliers == 2**31 - 100
+    for rows, at in ((x[:128], 0), (x[-64:], r.num_outliers)):
+        part = zs.compress_retiled(rows.contiguous(), window=window)
+        n = part.num_outliers
+        lo = at if at == 0 else at - n
+        assert torch.equal(r.exps[lo:lo + n], part.exps[:n])
+    assert not r.exps[r.num_outliers:].any()

@@ -653,17 +653,19 @@ constexpr int kCompactRecs = 8;
 constexpr int kCompactBuf = kCompactRecs * kExpFast + 16;  // group range + alignment
 
 // Bytes [E0, E1) of the stream from buf (byte 0 of it: stream byte E0 & ~3) by one
-// wave: whole dwords, byte stores only at the two ends.
+// wave: whole dwords, byte stores only at the two ends.  (Offsets from the first
+// dword: a stream may end less than a step short of 2^31.)
 __device__ __forceinline__ void put_range(const uint8_t* buf, uint8_t* exps, int E0, int E1) {
-  const int base = E0 & ~3;
-  for (int d = base + 4 * lane_id(); d < E1; d += 256) {
-    const uint32_t w = *reinterpret_cast<const uint32_t*>(buf + (d - base));
-    if (d >= E0 && d + 4 <= E1) {
-      *reinterpret_cast<uint32_t*>(exps + d) = w;
+  const int base = E0 & ~3, r0 = E0 - base, r1 = E1 - base;
+  uint8_t* out = exps + base;
+  for (int d = 4 * lane_id(); d < r1; d += 256) {
+    const uint32_t w = *reinterpret_cast<const uint32_t*>(buf + d);
+    if (d >= r0 && d + 4 <= r1) {
+      *reinterpret_cast<uint32_t*>(out + d) = w;
     } else {
 #pragma unroll
       for (int b = 0; b < 4; ++b)
-        if (d + b >= E0 && d + b < E1) exps[d + b] = (uint8_t)(w >> (8 * b));
+        if (d + b >= r0 && d + b < r1) out[d + b] = (uint8_t)(w >> (8 * b));
     }
   }
 }
@@ -704,17 +706,17 @@ __global__ __launch_bounds__(256) void rcompact_kernel(Src src, int M, int K,
 #pragma unroll
       for (int q = 0; q < kCompactRecs; ++q) {
         const int n = __builtin_amdgcn_readlane(nl, q);
-        const int e0 = __builtin_amdgcn_readlane(e0l, q);
+        const int e0 = __builtin_amdgcn_readlane(e0l, q) - base;
         if (q >= cnt || n == 0) continue;
         const int al = e0 & 3;
-        const int p0 = (e0 & ~3) + 4 * l;  // stream byte of this dword
+        const int p0 = (e0 & ~3) + 4 * l;  // buf byte of this dword
         const uint32_t v = al == 0 ? cur[q] : __builtin_amdgcn_alignbyte(cur[q], prev[q], 4 - al);
         if (p0 >= e0 && p0 + 4 <= e0 + n) {
-          *reinterpret_cast<uint32_t*>(buf + (p0 - base)) = v;
+          *reinterpret_cast<uint32_t*>(buf + p0) = v;
         } else {
 #pragma unroll
           for (int b = 0; b < 4; ++b)
-            if (p0 + b >= e0 && p0 + b < e0 + n) buf[p0 - base + b] = (uint8_t)(v >> (8 * b));
+            if (p0 + b >= e0 && p0 + b < e0 + n) buf[p0 + b] = (uint8_t)(v >> (8 * b));
         }
       }
       put_range(buf, exps, E0, E1);
