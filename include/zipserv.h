@@ -299,7 +299,9 @@ int zs_retiled_mm(void* stream, const uint8_t* d_fixed, const uint8_t* d_exps,
                   int N, int K, uint16_t* Reduction_Workspace, int Split_K);
 /* Name of the GEMM kernel that zs_retiled_mm, _fused and _fused_noalloc launch
  * for this shape on the current device (as a profiler shows it), NULL for a
- * shape they refuse.  No counterpart in the reference. */
+ * shape that zs_retiled_mm refuses.  2 * N * K > INT32_MAX runs as several
+ * blocks of X's rows; the name is that of the full ones.  No counterpart in the
+ * reference. */
 const char* zs_retiled_mm_kernel(int M, int N, int K, int split_k);
 /* zs_retiled_mm with the split-K reduction inside the GEMM kernel (no
  * counterpart in the reference, whose split-K always runs

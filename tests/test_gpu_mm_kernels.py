@@ -39,9 +39,24 @@ def test_kernel_of_every_shape_is_named():
         for N in (1, 16, 17, 500, 100000):
             for split_k in (1, 4):
                 name = lib.zs_retiled_mm_kernel(M, N, K, split_k)
-                assert (name is None) == (split_k > K // 64), (M, K, N, split_k)
-    for bad in ((63, 1, 64, 1), (64, 0, 64, 1), (64, 1, 32, 1), (64, 1, 64, 0)):
+                refused = split_k > K // 64 or M * N * split_k > 2 * (2**31 - 1)
+                assert (name is None) == refused, (M, K, N, split_k)
+    # the last two: 2^32 outputs, records of a band past 2^32 bytes
+    for bad in ((63, 1, 64, 1), (64, 0, 64, 1), (64, 1, 32, 1), (64, 1, 64, 0),
+                (28672, 200000, 64, 1), (64, 1, 64 * 3050403, 1)):
         assert lib.zs_retiled_mm_kernel(*bad) is None
+        # refused by the GEMM too, before any pointer is used
+        assert lib.zs_retiled_mm(None, 16, 16, 16, 0, 16, 16, *bad[:2], bad[2], 16, bad[3]) < 0
+
+
+def test_kernel_of_row_blocks_is_that_of_the_full_ones():
+    # 2 * N * K past INT32_MAX: blocks of 8176 rows
+    lib, K, full = zs.lib(), 131072, (2**31 - 1) // (2 * 131072) // 16 * 16
+    assert full == 8176
+    for N in (full + 100, 2 * full - 1, 3 * full):
+        for split_k in (1, 4):
+            assert lib.zs_retiled_mm_kernel(64, N, K, split_k) == \
+                lib.zs_retiled_mm_kernel(64, full, K, split_k)
 
 
 @pytest.mark.gpu

@@ -2756,25 +2756,38 @@ static const MmKernel& mm_kernel(int M, int N, int K, int split_k) {
 
 }  // namespace zs
 
+// Whether retiled_mm takes a shape.
+static int retiled_mm_shape(int M, int N, int K, int split_k) {
+  if (!shape_ok(M, K) || N <= 0 || split_k < 1 || split_k > K / 64) return ZS_E_INVAL;
+  // a band's records are addressed with 32-bit scalar offsets
+  if ((int64_t)(K / 64) * kRecBytes > (int64_t)UINT32_MAX) return ZS_E_OVERFLOW;
+  if ((int64_t)M * N * split_k > INT32_MAX * 2LL) return ZS_E_OVERFLOW;
+  return ZS_OK;
+}
+
+// Rows of X that one launch takes: the kernels address X with 32-bit byte
+// offsets, so that more than 2^31 bytes of it run as row blocks of X and Y, one
+// after another on the stream.  0: not even 16 rows fit (K > 2^26).
+static int retiled_mm_rows(int N, int K) {
+  if ((int64_t)N * K * 2 <= INT32_MAX) return N;
+  return (int)(INT32_MAX / (2LL * K)) / 16 * 16;
+}
+
 extern "C" const char* zs_retiled_mm_kernel(int M, int N, int K, int split_k) {
-  if (!shape_ok(M, K) || N <= 0 || split_k < 1 || split_k > K / 64) return nullptr;
-  return mm_kernel(M, N, K, split_k).name;
+  if (retiled_mm_shape(M, N, K, split_k) != ZS_OK) return nullptr;
+  const int rows = retiled_mm_rows(N, K);
+  return rows ? mm_kernel(M, rows, K, split_k).name : nullptr;
 }
 
 // Argument checks of retiled_mm that do not depend on the split-K buffers.
 static int retiled_mm_args(const uint8_t* d_fixed, const uint8_t* d_exps, const int32_t* d_eoff,
                            const uint16_t* B, const uint16_t* C, int M, int N, int K,
                            int split_k) {
-  if (!shape_ok(M, K) || N <= 0 || !d_fixed || !d_exps || !d_eoff || !B || !C) return ZS_E_INVAL;
+  if (!d_fixed || !d_exps || !d_eoff || !B || !C) return ZS_E_INVAL;
   if ((reinterpret_cast<uintptr_t>(d_fixed) & 15) || (reinterpret_cast<uintptr_t>(d_exps) & 15) ||
-      (reinterpret_cast<uintptr_t>(B) & 15) || (K % 8))
+      (reinterpret_cast<uintptr_t>(B) & 15))
     return ZS_E_INVAL;
-  const int KT = K / 64;
-  if (split_k < 1 || split_k > KT) return ZS_E_INVAL;
-  // a band's records are addressed with 32-bit scalar offsets
-  if ((int64_t)KT * kRecBytes > (int64_t)UINT32_MAX) return ZS_E_OVERFLOW;
-  if ((int64_t)M * N * split_k > INT32_MAX * 2LL) return ZS_E_OVERFLOW;
-  return ZS_OK;
+  return retiled_mm_shape(M, N, K, split_k);
 }
 
 // Split-K partial sums go to ws; with `counters` the GEMM kernel itself adds
@@ -2786,12 +2799,9 @@ static int retiled_mm(void* stream, const uint8_t* d_fixed, const uint8_t* d_exp
   if (chk != ZS_OK) return chk;
   if (split_k > 1 && !ws) return ZS_E_INVAL;
   const int KT = K / 64;
-  if ((int64_t)N * K * 2 > INT32_MAX) {
-    // The kernels address X with 32-bit byte offsets: run row blocks of X
-    // and Y that stay below 2^31 bytes, one after another on the stream.
-    const int rows = (int)(INT32_MAX / (2LL * K)) / 16 * 16;
-    // a row block of fewer than 16 rows would not fit either (K > 2^26)
-    if (rows < 16) return ZS_E_OVERFLOW;
+  const int rows = retiled_mm_rows(N, K);
+  if (rows == 0) return ZS_E_OVERFLOW;
+  if (rows < N) {
     for (int n0 = 0; n0 < N; n0 += rows) {
       const int st_ = retiled_mm(stream, d_fixed, d_exps, d_eoff, start_exp,
                                  B + (int64_t)n0 * K, C + (int64_t)n0 * M, M,
