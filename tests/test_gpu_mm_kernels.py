@@ -18,6 +18,9 @@ CASES = [("zs::rgemm_kernel<1, 1, 4, 4, 1>", 4160, 1088, 1, 2),
          ("zs::rgemm_kernel<1, 1, 8, 4, 1>", 320, 2560, 1, 1),
          ("zs::rgemm_kernel<1, 1, 8, 4, 2>", 320, 1088, 4, 3),
          ("zs::rgemm_kernel<1, 1, 8, 4, 4>", 64, 4096, 6, 4),
+         ("zs::rgemm_kernel<1, 1, 4, 4, 4>", 12288, 4096, 8, 1),
+         ("zs::rgemm_kernel<1, 1, 8, 4, 0>", 4096, 4096, 9, 2),
+         (WIDE % "1, 4, 4", 5120, 5120, 8, 2),
          ("zs::rgemm_kernel<2, 1, 4, 3, 0>", 4160, 512, 13, 2),
          ("zs::rgemm_kernel<2, 1, 8, 3, 0>", 1984, 512, 16, 4),
          (WIDE % "1, 4, 2", 4160, 512, 1, 4), (WIDE % "1, 4, 2", 8192, 1088, 9, 3),

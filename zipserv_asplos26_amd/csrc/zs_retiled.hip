@@ -2640,11 +2640,9 @@ using MmLaunch = hipError_t (*)(hipStream_t, const uint8_t*, const uint8_t*, con
 struct MmKernel {
   const char* name;
   MmLaunch launch;
-  // N > 16: 16-column blocks and rows of a workgroup, workgroups that fit a CU
+  // N > 16: 16-column blocks and rows of a workgroup, workgroups a CU that count
+  // as one round of the grid, fewest K tiles of a slice,
   int nb, rows, per_cu, min_kt;
-  // and its time in us: start + round per round of the grid, load per K tile of
-  // the workgroups that the busiest CU gets, mean per K tile of the mean over
-  // the CUs, alone per K tile where two fit a CU and it gets one
   // and its time in us: start, round per round of the grid, group per
   // workgroup that the busiest CU gets, load per K tile of those, mean per K tile
   // of the mean over the CUs, alone per K tile where two fit a CU and it gets one
@@ -2663,8 +2661,11 @@ struct MmKernel {
 // is taken.  The model's constants are a least-squares fit of relative error
 // over 915 (M, K, N = 17..500, split-K 1 / 2 / 4) points, every kernel timed at
 // each; its choice is on average 0.8% (at most 17%) over the fastest kernel, the
-// thresholds on M, N and split-K that it replaced 12.5% (at most 89%).  The
-// 128-row kernels of 2 and 4 blocks count 4% more than their fit, since in a near
+// thresholds on M, N and split-K that it replaced 12.5% (at most 89%).  Over 855
+// other points, with the weights read from HBM, it is 0.3% (at most 15%) over it and
+// 9% faster than the thresholds.  per_cu is part of the fit: two workgroups of <1,
+// 4, 4> and three of <2, 4, 2> fit a CU, but constants fitted with those figures
+// choose worse (0.34% over those 855 points instead of 0.28%).  The 128-row kernels of 2 and 4 blocks count 4% more than their fit, since in a near
 // tie the smaller tiles lose less, and three K phases take slices of >= 24 K
 // tiles (on 16 the uneven phases cost up to 6%).
 #define ZS_MM_WIDE(NB, PH) "zs::rgemm_wide_kernel<" #NB ", 4, " #PH ", 2>", launch_rwide<NB, 4, PH>, NB, 64
@@ -2703,7 +2704,7 @@ static float mm_time(const MmKernel& k, int M, int N, int kt, int split_k, int64
    {"zs::rgemm_kernel<" #F ", 1, " #W ", " #D ", 4>", launch_rgemm<F, 1, W>}}
 static const MmKernel kNarrow14[4] = ZS_MM_NARROW(1, 4, 4), kNarrow18[4] = ZS_MM_NARROW(1, 8, 4),
                       kNarrow24[4] = ZS_MM_NARROW(2, 4, 3), kNarrow28[4] = ZS_MM_NARROW(2, 8, 3);
-static const MmKernel kOneBlock4 = kWideKernels[0],
+static const MmKernel kOneBlock4 = {"zs::rgemm_wide_kernel<1, 4, 4, 2>", launch_rwide<1, 4, 4>},
                       kOneBlock2 = {"zs::rgemm_wide_kernel<1, 4, 2, 2>", launch_rwide<1, 4, 2>};
 
 static const MmKernel& mm_kernel(int M, int N, int K, int split_k) {
@@ -2723,27 +2724,34 @@ static const MmKernel& mm_kernel(int M, int N, int K, int split_k) {
   // them fits, two otherwise, from 4 <= N on grids of 7/8 of one per CU (each
   // X tile crosses L2 once per four bands: 8-24% faster than one band per
   // workgroup at N = 8 / 16 on such grids), and on 5/8 of one per CU for N > 8
-  // or slices of up to 64 K tiles (6144 x 4096, two slices: 18.6 -> 13.1 us at N =
-  // 16, 14.8 -> 13.0 at 8; 10240 x 8192, N = 16: 35.0 -> 31.8; not 128 of them:
-  // 8192 x 28672, N = 16 64.4 -> 98.6); short slices at any N, where a band's
+  // or slices of up to 40 K tiles (6144 x 4096, two slices: 16.8 -> 13.3 us at N =
+  // 16, 15.1 -> 13.2 at 8; 5120 x 5120, two slices of 40 tiles, N = 8: 18.0 -> 14.8;
+  // 10240 x 8192, N = 16: 36.5 -> 33.0; but 12288 x 4096, one slice of 64, N = 8: 17.0
+  // -> 19.1, 10240 x 8192, N = 8 28.0 -> 32.6); short slices at any N, where a band's
   // workgroup is mostly its start-up and, split, its arrival (10240 x 4096, N =
   // 1, four slices: 1.78x; 16384 x 512, N = 3: 1.9-2.3x; one slice of 32 K tiles
-  // of 20480 rows at N = 1 is 18% slower so).
+  // of 20480 rows at N = 1 is 18% slower so; split grids of a whole round, 14336 x
+  // 4096, two slices of 32 tiles, N = 1: 22.6 -> 20.5, but 10240 x 8192, two of 64:
+  // 29.6 -> 35.0).
   const int64_t wide = (int64_t)(M / 64) * split_k;
   const bool full = wide >= cus, most = wide * 8 >= cus * 5;
-  if ((N >= 4 && wide * 8 >= cus * 7) || (most && (N > 8 || (N > 4 && kt <= 64) || kt <= 16)) ||
+  if ((N >= 4 && wide * 8 >= cus * 7) || (most && (N > 8 || (N > 4 && kt <= 40) || kt <= 16)) ||
       (full && split_k > 1 && kt <= 36))
     return wide <= cus ? kOneBlock4 : kOneBlock2;
   // Otherwise workgroups of 8 K phases over one band, or two bands for N > 8
   // once the grid keeps at least 192 workgroups (half the X bytes per record,
-  // the cost that grows with N).  Workgroups of 4 waves (16 per CU, twice the
+  // the cost that grows with N; below 384 bands it takes slices of more than 32 K
+  // tiles or N > 12 too: 4096 x 14336, two slices, N = 9 24.3 -> 21.9 us, 4096 x 4096
+  // 10.9 -> 11.5, at N = 16 12.3 -> 12.2).  Workgroups of 4 waves (16 per CU, twice the
   // K tiles per wave) instead of 8 for N > 1 on >= 640 bands (1-5 us faster at
   // N = 8 / 16 on 10240, 14336 and 28672 rows, slower on smaller grids), for N
   // = 1 on >= 896 bands (14336 rows: 21.9 -> 19.6 us; 10240 rows are 0.6 us
   // slower with 4 waves), and on > 512 of them for slices of up to 16 K tiles.
   const bool w4 = M / 16 >= (N > 1 ? 640 : 896) || (kt <= 16 && (int64_t)(M / 16) * split_k > 512);
   const int xd = N <= 2 ? 1 : N <= 4 ? 2 : N <= 8 ? 3 : 0;
-  if (N > 8 && (int64_t)(M / 16) * split_k >= 384) return w4 ? kNarrow24[xd] : kNarrow28[xd];
+  if (N > 8 && (M / 16 >= 384 ||
+                ((int64_t)(M / 16) * split_k >= 384 && (kt > 32 || N > 12))))
+    return w4 ? kNarrow24[xd] : kNarrow28[xd];
   return w4 ? kNarrow14[xd] : kNarrow18[xd];
 }
 
