@@ -312,3 +312,17 @@ def test_zipgemm_rejects_bad_args(torch_cuda):
     X = to_torch_bf16(normal_bf16(rng, (4, 128)))
     with pytest.raises(zs.ZipServError):
         zs.zipgemm(c, X, split_k=3)  # split_k > K/64
+
+
+def test_stream_handle_with_and_without_torchs_private_function(torch_cuda, monkeypatch):
+    torch, codec = torch_cuda, zs.codec
+    side = torch.cuda.Stream()
+    want = [int(torch.cuda.current_stream().cuda_stream), int(side.cuda_stream)]
+    assert want[0] != want[1]
+    for private in (True, False):
+        if not private:
+            monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+        got = [codec._stream()]
+        with torch.cuda.stream(side):
+            got.append(codec._stream())
+        assert got == want

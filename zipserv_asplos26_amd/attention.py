@@ -247,7 +247,10 @@ def flash_attn_with_kvcache_zipserv(q, zipserv_k, zipserv_v, zipserv_num_heads_k
     with zipserv_k / zipserv_v).  q: (B, 1, H, D) or (B, H, D) bf16 on the GPU;
     seqlen_k: tokens per sequence held by the caches; cache_seqlens: optional
     int / int32 tensor [B] of valid lengths.  Returns out shaped like q (and
-    the natural-log softmax_lse [B, H] when asked)."""
+    the natural-log softmax_lse [B, H] when asked).  With num_splits == 0 the
+    splits of long sequences follow cache_seqlens, so the rounding of one
+    sequence's result may change with the others' lengths; num_splits > 0 cuts
+    every sequence alike."""
     torch = _torch()
     shape = q.shape
     q3 = _q3(q)

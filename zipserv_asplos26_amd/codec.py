@@ -166,9 +166,13 @@ def _dptr(t) -> int:
 def _stream() -> int:
     """The current device's current stream, without the Stream object that
     torch.cuda.current_stream() builds (2.9 -> 0.3 us of a call; zipgemm 9.7
-    -> 6.9 us, compressed decode attention 17.1 -> 13.7 us on the host)."""
+    -> 6.9 us, compressed decode attention 17.1 -> 13.7 us on the host), where
+    torch has that private function."""
     torch = _torch()
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return raw(torch.cuda.current_device())
 
 
 @dataclass
