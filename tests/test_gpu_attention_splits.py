@@ -100,3 +100,29 @@ def test_workspace_without_room_for_the_plan_keeps_equal_splits(torch_cuda, layo
     assert first <= B * splits
     assert not torch.equal(outs[0], outs[1])
     assert torch.equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("layout", ["by_kv_head", "token_major"])
+def test_replays_follow_the_lengths(torch_cuda, layout):
+    # a captured call reads the lengths, and makes its plan of them, on every replay
+    import zipserv_asplos26_amd.attention as za
+    torch = torch_cuda
+    B, T, Hkv, H = 6, 6000, 8, 32
+    q, kv, lens = _inputs(torch, layout, B, T, Hkv, H, True)
+    held = lens.clone()
+    call = lambda: za.flash_attn_with_kvcache_zipserv(q, *kv, Hkv, T, held)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for step in range(4):
+        held.copy_(lens.flip(0) if step % 2 else lens.clamp(max=1000 * (step + 1)))
+        graph.replay()
+        got = out.clone()
+        want = call()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))

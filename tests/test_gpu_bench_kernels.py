@@ -1,6 +1,6 @@
 """bench.py labels every timed launch with the kernel the library dispatches
-for its (M, N, K, split-K) (`bench.kernel_name`, a mirror of the dispatch in
-zs_retiled_mm).  Here the kernel that actually ran, as the HIP profiler
+for its (M, N, K, split-K) (`bench.kernel_name`, from zs_retiled_mm_kernel).
+Here the kernel that actually ran, as the HIP profiler
 records it, must carry that name, over one case of every dispatch branch."""
 import pytest
 

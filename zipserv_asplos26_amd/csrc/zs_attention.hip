@@ -332,7 +332,7 @@ __device__ __forceinline__ int kv_median(int rowbase, int med) {
 // LDS at the end (for small grids: kWpi x the waves without the cost of
 // kWpi x the global splits).
 // The re-tiled mode asks for three waves per SIMD: the compiler then keeps
-// the MFMA accumulators in ordinary VGPRs (140 in all, no spills) instead of
+// the MFMA accumulators in ordinary VGPRs (132 in all, no spills) instead of
 // splitting 135 VGPRs + 36 AGPRs, which allowed only two.
 // kBalanced: splits follow the lengths (instances of their own: with the plan's
 // code in every start-up, calls without a plan took 0.3-0.6 us longer).
@@ -1131,7 +1131,7 @@ static int attn_auto_splits(int batch, int heads_k, int seqlen_k, bool compresse
 }
 
 // Splits of the re-tiled mode, and whether a workgroup's four waves share one
-// item.  Three of its workgroups fit a CU (45 KB of LDS, 128 VGPRs), and one
+// item.  Three of its workgroups fit a CU (45 KB of LDS, 132 VGPRs), and one
 // full round of them is what is fast: 768 shared items, or 3072 of one wave
 // (the merge of four waves in LDS saves three quarters of the partial results,
 // 2-8% at equal rounds).  Grids of 2048 one-wave items, two thirds of a round,

@@ -1659,8 +1659,8 @@ __global__ __launch_bounds__(kSkWaves * 64, 6) void rgemm_sk_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// ZipGEMM over the re-tiled layout for wider batches (N > 16, and 4 <= N <= 16
-// on grids of at least 7/8 of a workgroup per CU).  Workgroup =
+// ZipGEMM over the re-tiled layout for wider batches, and for N <= 16 on grids of
+// 5/8 or 7/8 of a workgroup per CU or more (mm_kernel).  Workgroup =
 // BANDS*PH waves on one 16*BANDS-row tile x one split-K slice x 16*NB
 // columns; wave w decodes band w%BANDS of K tiles kb0 + PH*s + w/BANDS (PH
 // interleaved phases).  Each X tile (16*NB x 64) is loaded once per
